@@ -108,10 +108,10 @@ constexpr int TRACE_WORDS = 8;
 
 // Kernel arguments. v is the V buffer the kernel reads: the prep kernel's
 // V^T (contiguous, 128 rows of seq_k keys per KV head) or, for the tile that
-// reads V in its natural layout, the caller's v or its padded copy. seq_k is
-// the key length of the K and V buffers the
-// kernel reads (a multiple of its key block); keys at or past nk_valid are
-// zero padding and masked out of the softmax. lse (FP32 [B, Hq, Nq],
+// reads V in its natural layout, the caller's v or its copy. seq_k is
+// the key length the kernel works on (a multiple of its key block); keys at
+// or past nk_valid read as zeros (the buffer descriptors end there, the V^T
+// holds zeros) and are masked out of the softmax. lse (FP32 [B, Hq, Nq],
 // natural-log log-sum-exp of the scaled scores) may be null. stats, when not
 // null, receives the online-softmax statistics of every row after every key
 // block (capture mode): FP32 [4][seq_k / BN][B * Hq * Nq]
@@ -123,7 +123,7 @@ constexpr int TRACE_WORDS = 8;
 // (causal_off = 0 aligns the mask top-left, Nk - Nq bottom-right); a row that
 // sees no key gets O = 0 and lse = -inf. qs, ks, vs and os are the element
 // strides of q, of the K and natural-layout V buffers read (the caller's k
-// and v, or their padded contiguous copies) and of o. In split mode (splits >= 2) the kernel writes,
+// and v, or their contiguous copies) and of o. In split mode (splits >= 2) the kernel writes,
 // instead of o and lse, each part's O normalised by its own row sum into
 // opart (FP32 [splits][B * Hq * Nq][128]) and the part's natural-log
 // log-sum-exp into lpart (FP32 [splits][B * Hq * Nq]; -inf for a part in
@@ -200,8 +200,8 @@ __device__ __forceinline__ int vt_key_of_slot(int slot) {
 // Prep for the tiles that read V transposed: vt[kv][d][key0 + slot] =
 // v[kv][key0 + key(slot)][d], one 64-key group per workgroup; keys at or past
 // nk_valid become zeros. With kpad non-null the group's K rows are also
-// copied to kpad[kv][key0 + r] (zero rows past nk_valid), the padded K a
-// masked key tail reads. Grid (nk_pad / 64, B * Hkv), 256 threads; v and k
+// copied to kpad[kv][key0 + r] (zero rows past nk_valid), for a K whose rows
+// lie too far apart for 32-bit offsets (see rows_in_place). Grid (nk_pad / 64, B * Hkv), 256 threads; v and k
 // hold nk_valid keys per head with strides vs and ks, vt and kpad are
 // contiguous with nk_pad keys per head. It also resets the attention
 // kernel's tile counter.
@@ -247,12 +247,13 @@ __global__ void __launch_bounds__(256) fa_prep_kernel(const _Float16* __restrict
 }
 
 // Prep for the tile that reads V in its natural layout: resets the attention
-// kernel's tile counter and, for a ragged key tail (kpad non-null), writes
-// zero-padded copies of K and V: kpad[kv][key] and vpad[kv][key] hold the
+// kernel's tile counter and, for a K or V whose rows lie too far apart for
+// 32-bit offsets (kpad non-null, see rows_in_place), writes zero-padded
+// copies of both: kpad[kv][key] and vpad[kv][key] hold the
 // caller's rows for keys below nk_valid and zeros up to nk_pad, one 64-key
 // group per workgroup (grid (nk_pad / 64, B * Hkv), 256 threads; k and v hold
 // nk_valid keys per head with strides ks and vs, the copies are contiguous).
-// Without a tail the attention kernel reads the caller's k and v themselves,
+// Without copies the attention kernel reads the caller's k and v themselves,
 // and this kernel runs as one workgroup.
 __global__ void __launch_bounds__(256) fa_pad_kernel(const _Float16* __restrict__ k,
                                                      const _Float16* __restrict__ v,
@@ -295,7 +296,8 @@ __device__ __forceinline__ h4 lds_read_tr(const char* p) {
 
 // Raw-buffer descriptor (gfx9 layout: base address, stride 0, range in
 // bytes, 32-bit data format) for loads from `base`; the hardware returns
-// zeros for any lane whose offset lies at or past `bytes`.
+// zeros for any 32-bit word whose offset (per-lane plus scalar) lies at or
+// past `bytes`, also into LDS (direct-to-LDS loads write the zeros).
 __device__ __forceinline__ i32x4 buffer_rsrc(const void* base, int bytes) {
   const uint64_t a = reinterpret_cast<uint64_t>(base);
   return i32x4{(int)(uint32_t)a, (int)(uint32_t)(a >> 32), bytes, 0x00020000};
@@ -761,11 +763,12 @@ __device__ __forceinline__ void fa_pp_tile(const FaArgs& args, const int tile, c
     }
   }
   // The loads are buffer loads through one descriptor per operand (base =
-  // this KV head's K or V, range = the bytes its seq_k rows span, so the
+  // this KV head's K or V, range = the bytes its nk_valid rows span, so the
   // hardware bounds-checks every lane): the per-lane offset is dma_off, the
-  // block offset a wave-uniform scalar (see dma_to_lds).
-  const i32x4 krsrc = buffer_rsrc(kp + (size_t)kb0 * BN * args.ks.n, (seq_k - kb0 * BN - 1) * krow + HD * 2);
-  const i32x4 vrsrc = VNAT ? buffer_rsrc(vp + (size_t)kb0 * BN * args.vs.n, (seq_k - kb0 * BN - 1) * vrow + HD * 2)
+  // block offset a wave-uniform scalar (see dma_to_lds). A ragged last block
+  // reaches past the range, and its missing rows arrive in LDS as zeros.
+  const i32x4 krsrc = buffer_rsrc(kp + (size_t)kb0 * BN * args.ks.n, (nk_valid - kb0 * BN - 1) * krow + HD * 2);
+  const i32x4 vrsrc = VNAT ? buffer_rsrc(vp + (size_t)kb0 * BN * args.vs.n, (nk_valid - kb0 * BN - 1) * vrow + HD * 2)
                            : buffer_rsrc(vp + kb0 * BN, seq_k * (HD * 2) - kb0 * (BN * 2));
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
   // DMA instruction m of this wave for K block kb -> ring slot ks and V
@@ -1422,20 +1425,24 @@ int select_tile(const fa_problem* p, const TileConfig** out) {
   return FA_OK;
 }
 
-// Key length of the K and V buffers the attention kernel reads: Nk itself
-// when the tile's key block divides it, else Nk rounded up to a whole block
-// (64 or 128 keys, both whole prep groups), zero-padded by the prep kernel:
-// it then writes padded copies of K and (natural-V tile) V into the
-// workspace. The V^T tiles always read the prep kernel's V^T, the natural-V
-// tile the caller's v (or its padded copy). The last block holds at least
-// one real key.
+// Key length the attention kernel works on: Nk itself when the tile's key
+// block divides it, else Nk rounded up to a whole block (64 or 128 keys, both
+// whole prep groups). The V^T tiles always read the prep kernel's V^T, whose
+// rows end in zeros; K, and V for the natural-V tile, are read where they lie
+// also with a ragged tail (the buffer descriptors end at the last real row
+// and the loads past it give zeros), except where their rows span too much
+// for that (rows_in_place): then the prep kernel writes padded copies into
+// the workspace, which is sized for them whenever there is a tail, as the
+// strides are not known when it is sized. The last block holds at least one
+// real key.
 struct KeyLayout {
   int64_t nk_pad;
-  bool pad;              // ragged key tail: the kernel reads padded copies
+  bool pad;              // ragged key tail
   bool vnat;             // the tile reads V in its natural layout
   uint64_t head_bytes;   // one copy of K, V or V^T: B * Hkv * nk_pad * 128 * 2
-  // Workspace: V^T (V^T tiles), the padded K, the padded V (natural-V tile),
-  // then the attention kernel's tile counter in a 256-byte slot of its own.
+  // Workspace: V^T (V^T tiles), room for the padded K and (natural-V tile) the
+  // padded V, then the attention kernel's tile counter in a 256-byte slot of
+  // its own.
   int copies() const { return (vnat ? 0 : 1) + (pad ? (vnat ? 2 : 1) : 0); }
   uint64_t counter_offset() const { return copies() * head_bytes; }
   uint64_t workspace_bytes() const { return counter_offset() + kCounterBytes; }
@@ -1627,6 +1634,18 @@ Strides contiguous(int64_t heads, int64_t seq) { return Strides{heads * seq * HD
 
 Strides strides_of(const int64_t* s) { return Strides{s[0], s[1], s[2]}; }
 
+// Whether a buffer of nk_pad key rows n elements apart, of which the last may
+// lie past the tensor, is addressed with 32-bit byte offsets (buffer loads
+// check every offset against the real rows; the offsets of the rows past
+// them must not wrap). A ragged tail is then read in place; reading it
+// through padded copies costs a pass that reads and writes all of K and V
+// (B=8 Hq=64 Hkv=8 Nq=1 Nk=8005: 94 us of copies before a 51 us attention
+// kernel, 147 us per forward; in place 54 us).
+bool rows_in_place(int64_t n, int64_t nk_pad) {
+  const int64_t lim = (int64_t)1 << 30;
+  return n < lim && n * nk_pad < lim;
+}
+
 // Caller strides must keep every 128-element row 16-byte aligned and rows
 // apart (n >= 128); the K rows of one head, and its V rows if the tile reads
 // them in place (natural-V tile), must span less than 2^31 bytes (32-bit
@@ -1765,11 +1784,13 @@ int launch(const fa_problem* p, const fa_strides* strides, const void* q, const 
 
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   // Workspace: [V^T] [padded K] [padded V] counter, as the layout has them.
+  const bool copies = lay.pad && !(rows_in_place(ks.n, lay.nk_pad) &&
+                                   (!lay.vnat || rows_in_place(vs.n, lay.nk_pad)));
   _Float16* ws = static_cast<_Float16*>(workspace);
   const uint64_t head_elems = lay.head_bytes / sizeof(_Float16);
   _Float16* vt = lay.vnat ? nullptr : ws;
-  _Float16* kpad = lay.pad ? ws + (lay.vnat ? 0 : head_elems) : nullptr;
-  _Float16* vpad = lay.pad && lay.vnat ? kpad + head_elems : nullptr;
+  _Float16* kpad = copies ? ws + (lay.vnat ? 0 : head_elems) : nullptr;
+  _Float16* vpad = copies && lay.vnat ? kpad + head_elems : nullptr;
   int* next_tile = reinterpret_cast<int*>(static_cast<char*>(workspace) + lay.counter_offset());
 
   // hipLaunchKernel returns the status of this launch alone; errors left
@@ -1792,7 +1813,7 @@ int launch(const fa_problem* p, const fa_strides* strides, const void* q, const 
     void* vt_args[] = {&kk, &vv, &vt, &kpad, &nk_valid, &nk_pad, &heads_kv, &ks, &vs, &next_tile};
     void* pad_args[] = {&kk, &vv, &kpad, &vpad, &nk_valid, &nk_pad, &heads_kv, &ks, &vs, &next_tile};
     const dim3 groups((unsigned)(lay.nk_pad / PAD_GROUP), (unsigned)(p->batch * p->heads_kv));
-    // The natural-V tile without a key tail needs the pad kernel only for
+    // The natural-V tile without copies needs the pad kernel only for
     // the counter, which a launch of at most one work item per CU does not
     // use (fa_pp_body): then nothing runs before the attention kernel.
     const bool direct = grid_size(p) * splits <= (uint64_t)cus;
@@ -1800,16 +1821,16 @@ int launch(const fa_problem* p, const fa_strides* strides, const void* q, const 
     if (!lay.vnat)
       ok = hipLaunchKernel(reinterpret_cast<const void*>(&fa_prep_kernel), groups, dim3(256),
                            vt_args, 0, st) == hipSuccess;
-    else if (lay.pad || !direct)
+    else if (copies || !direct)
       ok = hipLaunchKernel(reinterpret_cast<const void*>(&fa_pad_kernel),
-                           lay.pad ? groups : dim3(1, 1), dim3(256), pad_args, 0, st) == hipSuccess;
+                           copies ? groups : dim3(1, 1), dim3(256), pad_args, 0, st) == hipSuccess;
     if (!ok) return FA_ERR_LAUNCH;
   }
 
   FaArgs args;
   args.q = static_cast<const _Float16*>(q);
-  args.k = lay.pad ? kpad : static_cast<const _Float16*>(k);
-  args.v = !lay.vnat ? vt : lay.pad ? vpad : static_cast<const _Float16*>(v);
+  args.k = copies ? kpad : static_cast<const _Float16*>(k);
+  args.v = !lay.vnat ? vt : copies ? vpad : static_cast<const _Float16*>(v);
   args.o = static_cast<_Float16*>(o);
   args.lse = ex.lse;
   args.stats = ex.stats;
@@ -1829,8 +1850,8 @@ int launch(const fa_problem* p, const fa_strides* strides, const void* q, const 
   args.c = (float)((double)p->scale * LOG2E);
   args.qs = qs;
   args.os = os;
-  args.ks = lay.pad ? contiguous(p->heads_kv, lay.nk_pad) : ks;
-  args.vs = lay.pad || !lay.vnat ? contiguous(p->heads_kv, lay.nk_pad) : vs;
+  args.ks = copies ? contiguous(p->heads_kv, lay.nk_pad) : ks;
+  args.vs = copies || !lay.vnat ? contiguous(p->heads_kv, lay.nk_pad) : vs;
   void* attn_args[] = {&args};
   // One workgroup per CU (the LDS ring leaves room for no second one), never
   // more workgroups than work items.

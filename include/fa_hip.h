@@ -121,9 +121,11 @@ typedef struct fa_problem {
  * Bytes of device workspace fa_fwd() needs for problem *p: 256 bytes for the
  * counter the kernel's workgroups take query tiles from, plus, for a tile
  * that reads V^T (see V layouts above), V^T (B * Hkv * Nk' * 256 bytes), and,
- * with a ragged key tail, zero-padded copies to a whole key block of the
- * selected tile (Nk' keys) of k (V^T tiles) or of k and v (pp_n128_r2_vnat),
- * B * Hkv * Nk' * 256 bytes each. pp_n128_r2_vnat without a key tail reads k
+ * with a ragged key tail, room for zero-padded copies to a whole key block of
+ * the selected tile (Nk' keys) of k (V^T tiles) or of k and v
+ * (pp_n128_r2_vnat), B * Hkv * Nk' * 256 bytes each (written only when the
+ * rows of k or v lie so far apart that Nk' of them span 2 GiB or more;
+ * otherwise a ragged tail is read in place). pp_n128_r2_vnat without a key tail reads k
  * and v where they lie and needs the 256-byte counter alone. Replaces phase 1 of the
  * reference's operator call,
  * aclnn<Op>GetWorkspaceSize (backends/cce_fa_nk_nz_vector_fp32_v5_sumpack/
@@ -276,7 +278,7 @@ const char* fa_kernel_name(int32_t kernel);
  * device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc). No counterpart in the reference. The
  * workspace (fa_fwd_workspace_bytes(): the tile counter, V^T for the V^T
- * tiles, padded copies for a ragged key tail) lives in a static device array
+ * tiles, the room for a ragged key tail's copies) lives in a static device array
  * of FA_NOALLOC_SCRATCH_BYTES per GPU, which the library holds from module
  * load until the process ends; problems whose fa_fwd_workspace_bytes()
  * exceeds it fail with FA_ERR_SCRATCH before any work is enqueued (64 MiB +
