@@ -1326,6 +1326,305 @@ __device__ __forceinline__ void fa_pp_body(const FaArgs& args) {
   }
 }
 
+// The few-row kernel: split mode for row sequences that fill at most
+// kRowTilesMax 32-row tiles per KV head (decode, a few tokens behind a cache).
+// There the forward reads every key once and is bound by that read, so the
+// kernel is laid out for bytes in flight and no waiting: a work item is one
+// tile of 32 rows and one part of its keys, and each of the 8 waves takes
+// every eighth 32-key block of the part for itself -- its own LDS slots (8 KiB
+// of K, 8 KiB of V), its own softmax statistics and O -- so the key loop has
+// no barrier. A wave loads K(j + 1) as soon as K(j) is in registers and
+// V(j + 1) after the PV products of block j: up to 128 KiB per CU in flight.
+// The 8 waves' results are combined through LDS at the end, so a part hands
+// the merge kernel one row, not eight.
+// Against the 256-row ping-pong body, of whose 8 waves a decode tile uses one
+// and whose key blocks follow each other through two barriers each, per
+// forward: Hq=12 Hkv=1, 16 rows behind 50001 keys 25.1 -> 20.2 us; B=8 Hq=64
+// Hkv=8, one row behind 8005 keys 54.6 -> 52.8 us (262 MB, 5.0 TB/s); one row
+// behind 4099 keys 11.4 + 3.6 -> 7.1 + 3.6 us of kernels (attention + merge),
+// behind 131072 keys 15.6 + 6.4 -> 15.1 + 5.7 us (64 MiB at 4.4 TB/s; a large
+// copy reaches 4.7).
+//
+// LDS rows are 256 bytes with no pad; K stores chunk c of row r at position
+// c ^ (r % 16), so the rows an operand read takes one chunk column from lie
+// in different banks; V uses the natural-V tile's swizzle.
+constexpr int RT = 32;                      // query rows per tile
+constexpr int RSUB = 32;                    // keys per block of a wave
+constexpr int RSLOT = RSUB * HD * 2;        // bytes of a K or V block
+constexpr int kRowsLds = 8 * 2 * RSLOT + 2 * 8 * RT * 4;   // slots (reused for O), then m and l
+
+template <int N>
+__device__ __forceinline__ void wait_loads() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+// Every LDS read this wave has issued has returned: its slot can be refilled.
+__device__ __forceinline__ void wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+
+template <bool ACC16, bool PACKED>
+__device__ __forceinline__ void fa_rows_body(const FaArgs& args) {
+  constexpr float TAU = ACC16 ? 0.f : 8.f;
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, l32 = lane & 31, hf = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int group = args.group, heads_kv = args.heads_q / group;
+  const int seq_r = PACKED ? args.seq_q * group : args.seq_q;
+  const int tiles_q = (seq_r + RT - 1) / RT;
+  // Workgroup -> (KV head, part, tile). Consecutive workgroups go to
+  // different dies; the tiles that read the same keys (T per KV head and
+  // part) are given to one die, so its L2 fetches those keys once.
+  const int T = PACKED ? tiles_q : tiles_q * group;
+  const int slot = (int)blockIdx.x >> 3;
+  const int unit = slot / T * 8 + ((int)blockIdx.x & 7);
+  const int tile_in = slot % T;
+  const int splits = args.splits;
+  if (unit >= args.tiles / T * splits) return;
+  const int kv = unit / splits, split = unit - kv * splits;
+  const int b = kv / heads_kv, hk = kv - b * heads_kv;
+  const int qt = tile_in % tiles_q;
+  const int hs = PACKED ? hk : hk * group + tile_in / tiles_q;
+  auto head_of = [&](int r) { return PACKED ? hk * group + r % group : hs; };
+  auto pos_of = [&](int r) { return PACKED ? r / group : r; };
+  const int row = qt * RT + l32;
+  const bool row_ok = row < seq_r;
+  const int rowc = row_ok ? row : seq_r - 1;
+  const size_t rows_all = (size_t)(args.tiles / T) * group * args.seq_q;   // B * Hq * Nq
+  const size_t grow = ((size_t)b * args.heads_q + head_of(rowc)) * args.seq_q + pos_of(rowc);
+  const size_t part = (size_t)split * rows_all + grow;
+
+  // The part's keys [k0, kend), as the ping-pong body cuts them (whole
+  // 128-key blocks), up to the last key the tile's last row sees.
+  const int nbt = args.seq_k / 128;
+  const int k0 = (int)((int64_t)split * nbt / splits) * 128;
+  int kend = min((int)((int64_t)(split + 1) * nbt / splits) * 128, args.nk_valid);
+  int klim = args.nk_valid - 1, klim_w = klim;
+  if (args.causal) {
+    klim = min(klim, pos_of(row) + args.causal_off);
+    klim_w = min(klim_w, pos_of(qt * RT) + args.causal_off);
+    kend = min(kend, pos_of(min(qt * RT + RT, seq_r) - 1) + 1 + args.causal_off);
+  }
+  klim -= k0;
+  klim_w -= k0;
+  const int nsub = kend <= k0 ? 0 : (kend - k0 + RSUB - 1) / RSUB;
+  if (nsub == 0) {
+    // No row of the tile sees a key of this part: weight 0 in the merge.
+    if (!row_ok || wave) return;
+    if (hf == 0) args.lpart[part] = -INFINITY;
+    const float4 zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < 16; ++i) *reinterpret_cast<float4*>(args.opart + part * HD + 8 * i + 4 * hf) = zero;
+    return;
+  }
+
+  // A load instruction fills 4 rows: lane l brings row l / 16, the chunk its
+  // swizzled position holds (K's swizzle repeats every 4 instructions).
+  // Blocks past the part's end are loaded from past the descriptors' range:
+  // they fetch nothing, and every block issues the same 8 loads, which keeps
+  // the wait counts constant.
+  const int krow = (int)(args.ks.n * 2), vrow = (int)(args.vs.n * 2);
+  const int krange = (args.nk_valid - k0 - 1) * krow + HD * 2;
+  const int vrange = (args.nk_valid - k0 - 1) * vrow + HD * 2;
+  const i32x4 krsrc = buffer_rsrc(row_at(args.k, args.ks, b, hk, k0), krange);
+  const i32x4 vrsrc = buffer_rsrc(row_at(args.v, args.vs, b, hk, k0), vrange);
+  const int lr = lane >> 4;
+  int koff[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) koff[i] = lr * krow + ((lane & 15) ^ (4 * i + lr)) * 16;
+  const int voff = lr * vrow + ((lane & 15) ^ (4 * lr)) * 16;
+  char* kslot = lds + wave * 2 * RSLOT;
+  char* vslot = kslot + RSLOT;
+  const uint32_t kdst = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)kslot;
+  const uint32_t vdst = kdst + RSLOT;
+  auto load_k = [&](int sub) {
+    const int key = sub * RSUB;
+#pragma unroll
+    for (int i = 0; i < RSUB / 4; ++i)
+      dma_to_lds(krsrc, kdst + i * 1024, koff[i & 3], sub < nsub ? (key + 4 * i) * krow : krange);
+  };
+  auto load_v = [&](int sub) {
+    const int key = sub * RSUB;
+#pragma unroll
+    for (int i = 0; i < RSUB / 4; ++i)
+      dma_to_lds(vrsrc, vdst + i * 1024, voff, sub < nsub ? (key + 4 * i) * vrow : vrange);
+  };
+
+  h8 qf[8];
+#pragma unroll
+  for (int kk = 0; kk < 8; ++kk)
+    qf[kk] = *reinterpret_cast<const h8*>(row_at(args.q, args.qs, b, head_of(rowc), pos_of(rowc)) +
+                                          kk * 16 + hf * 8);
+  load_k(wave);
+  load_v(wave);
+  // The compiler waits for its own loads here, before the key loop.
+#pragma unroll
+  for (int kk = 0; kk < 8; ++kk) asm volatile("" ::"v"(qf[kk]));
+
+  const float c = args.c;
+  f32x16 acc[4];
+#pragma unroll
+  for (int dt = 0; dt < 4; ++dt) acc[dt] = f32x16{};
+  float m = NEG_BIG, lsum = 0.f;
+  auto round_acc_fp16 = [&]() {
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[dt][i] = (float)(_Float16)acc[dt][i];
+  };
+  // Operand addresses: K chunk 2kk + hf of row l32; V as in the natural-V
+  // tile (fa_pp_tile).
+  const int k_lane = l32 * 256 + ((hf ^ (l32 & 15)) << 4);
+  int v_lane[4];
+#pragma unroll
+  for (int dt = 0; dt < 4; ++dt) {
+    const int e = (lane & 15) >> 2;
+    v_lane[dt] = (4 * hf + e) * 256 + (4 * (dt ^ e) + 2 * (lr & 1) + ((lane & 3) >> 1)) * 16 +
+                 (lane & 1) * 8;
+  }
+
+  int j = 0;
+  for (int sub = wave; sub < nsub; sub += 8, ++j) {
+    if constexpr (ACC16)                    // O is FP16 after every 512 keys of the wave
+      if (j > 0 && j % (512 / RSUB) == 0) round_acc_fp16();
+    wait_loads<8>();                        // K(j) has landed; V(j) may be in flight
+    f32x16 sc = f32x16{};
+#pragma unroll
+    for (int kk = 0; kk < 8; ++kk)
+      sc = mfma32(*reinterpret_cast<const h8*>(kslot + (k_lane ^ (kk << 5))), qf[kk], sc);
+    wait_lds();
+    load_k(sub + 8);
+    const int key0 = sub * RSUB;
+    if (key0 + RSUB - 1 > klim_w) {         // some row of the tile does not see the whole block
+      const int lim = klim - key0 - 4 * hf;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const float d = (float)(8 * (r >> 2) + (r & 3) - lim);
+        sc[r] = __builtin_fmaf(__builtin_amdgcn_fmed3f(d, 0.f, 1.f), MASKED, sc[r]);
+      }
+    }
+    float mv[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) mv[r] = sc[r];
+#pragma unroll
+    for (int n = 16; n > 1; n = (n + 2) / 3) {
+#pragma unroll
+      for (int i = 0; 3 * i < n; ++i) {
+        float x = mv[3 * i];
+        if (3 * i + 1 < n) x = smax(x, mv[3 * i + 1]);
+        if (3 * i + 2 < n) x = smax(x, mv[3 * i + 2]);
+        mv[i] = x;
+      }
+    }
+    const float mx = half_max(mv[0]);
+    const bool need = (mx - m) * c > TAU;
+    if (__builtin_amdgcn_ballot_w64(need)) {
+      const float mnew = need ? smax(m, mx) : m;
+      const float alpha = __builtin_amdgcn_exp2f((m - mnew) * c);
+      m = mnew;
+      lsum *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt) acc[dt] *= alpha;
+    }
+    const float mc = m * c;
+    float ls[2] = {0.f, 0.f};
+    h8 p[2];
+#pragma unroll
+    for (int g2 = 0; g2 < 2; ++g2)
+#pragma unroll
+      for (int e = 0; e < 8; e += 2) {
+        const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[8 * g2 + e], c, -mc));
+        const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[8 * g2 + e + 1], c, -mc));
+        const h2 pr = {(_Float16)p0, (_Float16)p1};
+        p[g2][e] = pr[0];
+        p[g2][e + 1] = pr[1];
+        ls[0] = add_f16<0>(ls[0], pr);
+        ls[1] = add_f16<1>(ls[1], pr);
+      }
+    lsum += ls[0] + ls[1];
+    wait_loads<8>();                        // V(j) has landed; K(j + 1) may be in flight
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt) {
+        const char* at = vslot + v_lane[dt] + ks * 16 * 256;
+        const h8 a = __builtin_shufflevector(lds_read_tr(at), lds_read_tr(at + 8 * 256), 0, 1, 2, 3, 4,
+                                             5, 6, 7);
+        acc[dt] = mfma32(a, p[ks], acc[dt]);
+      }
+    wait_lds();
+    load_v(sub + 8);
+  }
+  if constexpr (ACC16) round_acc_fp16();
+
+  // Combine the waves through LDS: once its loads have landed, a wave's O
+  // goes to its own 16 KiB of slots, 512-byte rows with chunk c of row r at
+  // position c ^ r, and its m and l behind all slots.
+  wait_loads<0>();
+  float* st_m = reinterpret_cast<float*>(lds + 8 * 2 * RSLOT);
+  float* st_l = st_m + 8 * RT;
+  const float l = half_sum(lsum);
+  if (hf == 0) {
+    st_m[wave * RT + l32] = m;
+    st_l[wave * RT + l32] = l;
+  }
+  if (row_ok) {
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const float4 val = {acc[dt][4 * g], acc[dt][4 * g + 1], acc[dt][4 * g + 2], acc[dt][4 * g + 3]};
+        *reinterpret_cast<float4*>(kslot + l32 * 512 + (((dt * 8 + 2 * g + hf) ^ l32) << 4)) = val;
+      }
+  }
+  __syncthreads();
+  // 16 threads per row, 8 dims each: chunks t and t + 16.
+  const int r = tid >> 4, t = tid & 15;
+  const int orow = qt * RT + r;
+  if (orow >= seq_r) return;
+  float mw[8], M = NEG_BIG;
+#pragma unroll
+  for (int w = 0; w < 8; ++w) {
+    mw[w] = st_m[w * RT + r];
+    M = smax(M, mw[w]);
+  }
+  float L = 0.f;
+  float4 o0 = {0.f, 0.f, 0.f, 0.f}, o1 = o0;
+#pragma unroll
+  for (int w = 0; w < 8; ++w) {
+    const float f = __builtin_amdgcn_exp2f((mw[w] - M) * c);
+    L = __builtin_fmaf(f, st_l[w * RT + r], L);
+    const char* base = lds + w * 2 * RSLOT + r * 512;
+    const float4 a0 = *reinterpret_cast<const float4*>(base + ((t ^ r) << 4));
+    const float4 a1 = *reinterpret_cast<const float4*>(base + (((t + 16) ^ r) << 4));
+    o0.x = __builtin_fmaf(f, a0.x, o0.x);
+    o0.y = __builtin_fmaf(f, a0.y, o0.y);
+    o0.z = __builtin_fmaf(f, a0.z, o0.z);
+    o0.w = __builtin_fmaf(f, a0.w, o0.w);
+    o1.x = __builtin_fmaf(f, a1.x, o1.x);
+    o1.y = __builtin_fmaf(f, a1.y, o1.y);
+    o1.z = __builtin_fmaf(f, a1.z, o1.z);
+    o1.w = __builtin_fmaf(f, a1.w, o1.w);
+  }
+  const float inv = L > 0.f ? 1.f / L : 0.f;
+  const size_t opos = (size_t)split * rows_all +
+                      ((size_t)b * args.heads_q + head_of(orow)) * args.seq_q + pos_of(orow);
+  float* dst = args.opart + opos * HD;
+  *reinterpret_cast<float4*>(dst + 4 * t) = float4{o0.x * inv, o0.y * inv, o0.z * inv, o0.w * inv};
+  *reinterpret_cast<float4*>(dst + 64 + 4 * t) = float4{o1.x * inv, o1.y * inv, o1.z * inv, o1.w * inv};
+  if (t == 0) args.lpart[opos] = (__builtin_amdgcn_logf(L) + M * c) * LN2;
+}
+
+template <bool PACKED>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+hip_fa_fp32acc_rows_kernel(FaArgs args) {
+  fa_rows_body<false, PACKED>(args);
+}
+
+template <bool PACKED>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+hip_fa_fp16acc_rows_kernel(FaArgs args) {
+  fa_rows_body<true, PACKED>(args);
+}
+
 // LDS bytes the ping-pong body needs for BN-key blocks (a ring of NS K and
 // NS V or V^T blocks with padded rows).
 constexpr int pp_lds_bytes(int bn, int ns, bool vnat) {
@@ -1513,6 +1812,27 @@ RowLayout row_layout(const fa_problem* p) {
 // Query tiles of one attention launch (one per 256 rows of a row sequence).
 uint64_t grid_size(const fa_problem* p) { return (uint64_t)row_layout(p).tiles(); }
 
+// The few-row kernel (fa_rows_body) runs split launches of the automatic tile
+// choice whose rows fill at most kRowTilesMax of its 32-row tiles per KV head:
+// every tile streams the part's keys for itself, so beyond a few tiles the
+// 256-row tiles, which read them once for eight times the rows, are cheaper.
+constexpr int64_t kRowTilesMax = 8;
+int64_t row_tiles(const fa_problem* p) {    // 32-row tiles of the launch
+  const RowLayout rl = row_layout(p);
+  return rl.seqs * ((rl.rows + RT - 1) / RT);
+}
+bool few_rows(const fa_problem* p, int splits) {
+  const int64_t kv_heads = p->batch * p->heads_kv;
+  const int64_t rows = rows_per_kv_head(p);
+  return p->kernel == 0 && rows > 0 && rows <= kNaturalVRows &&
+         row_tiles(p) <= kRowTilesMax * kv_heads &&
+         row_tiles(p) * splits < ((int64_t)1 << 22);   // its grid is not persistent
+}
+const attn_fn kRowsFn[2][2] = {   // [packed][acc]
+    {&hip_fa_fp32acc_rows_kernel<false>, &hip_fa_fp16acc_rows_kernel<false>},
+    {&hip_fa_fp32acc_rows_kernel<true>, &hip_fa_fp16acc_rows_kernel<true>},
+};
+
 // Split mode's partial results, after the tile counter in the workspace:
 // the parts' log-sum-exp (FP32 [splits][R], R = B * Hq * Nq) from a 256-byte
 // boundary, then their O (FP32 [splits][R][128]).
@@ -1596,6 +1916,35 @@ double split_cost(const fa_problem* p, const TileConfig* tile, const KeyLayout& 
   return t;
 }
 
+// Modelled duration (us) of a split launch of the few-row kernel with s parts,
+// or, s = 1, of the one-pass kernel in its place. Fitted to part-count sweeps
+// (12 rows behind 4099 to 131072 keys, 192 and 256 rows behind 50001, batches
+// of 64 to 256 tiles): a workgroup's first 256 keys cost 7 us from launch to
+// its result, each further 256 the latency of one block (1.25 us), or, with
+// many workgroups streaming, the time memory (4.7 TB/s over the keys read
+// once) or the L2s (17 TB/s over all of them) take for all workgroups' 128
+// KiB; a CU's later workgroups 5.5 us and their rounds; the merge
+// 3.4 us and 9 ns a part, plus its bytes. The one-pass kernel takes about 1.5
+// us per 128 keys with one wave at work.
+double few_rows_cost(const fa_problem* p, const KeyLayout& lay, int s, int cus) {
+  const double nbt = (double)(lay.nk_pad / 128);
+  const double kv_heads = (double)(p->batch * p->heads_kv);
+  const double round_bytes = 2.0 * 256 * HD * sizeof(_Float16);
+  if (s == 1) {
+    const double tiles = (double)grid_size(p);
+    const double read = std::min(tiles, (double)cus) * kv_heads / tiles * round_bytes / 2 / 4.7e6;
+    return ceil(tiles / cus) * (6.0 + std::max((nbt + 1) * 1.54, nbt * read));
+  }
+  const double items = (double)row_tiles(p) * s, active = std::min(items, (double)cus);
+  const double share = (double)row_tiles(p) / kv_heads;      // tiles that read the same keys
+  const double rounds = ceil(ceil(nbt / s) / 2);
+  const double per_round =
+      std::max(1.25, std::max(active / share * round_bytes / 4.7e6, active * round_bytes / 17e6));
+  const double rows = (double)(p->batch * p->heads_q) * p->seq_q;
+  return 7.0 + (rounds - 1) * per_round + (ceil(items / cus) - 1) * (5.5 + rounds * per_round) + 3.4 +
+         0.009 * s + rows * s * (HD * 4.0 + 4.0) / 4e6;
+}
+
 // Effective split count for a requested one: 0 picks the count with the
 // shortest modelled launch (splitting only when that beats one pass over the
 // keys by 10 %: tiles must leave CUs idle), n >= 1 is clamped to the tile's
@@ -1607,7 +1956,19 @@ int resolve_splits(const fa_problem* p, const TileConfig* tile, const KeyLayout&
   int s = (int)std::min<int64_t>(requested, nbt);
   if (requested == 0) {
     s = 1;
-    if (grid_size(p) < 2 * (uint64_t)cus) {
+    if (few_rows(p, kAutoSplitMax)) {
+      // The counts that change a workgroup's 256-key rounds, in steps of a quarter.
+      double best = few_rows_cost(p, lay, 1, cus);
+      for (int64_t rounds = 1; 2 * rounds < nbt; rounds += 1 + rounds / 4) {
+        const int64_t n = (nbt + 2 * rounds - 1) / (2 * rounds);
+        if (n > kAutoSplitMax) continue;
+        const double t = few_rows_cost(p, lay, (int)n, cus);
+        if (t < best) {
+          best = t;
+          s = (int)n;
+        }
+      }
+    } else if (grid_size(p) < 2 * (uint64_t)cus) {
       double best = 0.9 * split_cost(p, tile, lay, 1, cus);
       auto consider = [&](int c) {
         if (c > nbt) return;
@@ -1670,16 +2031,18 @@ int check_strides(const fa_problem* p, const fa_strides* s, const KeyLayout& lay
 // scratch addresses of fa_fwd_noalloc are the library's only host state;
 // setting either twice (two threads racing on a first call) is harmless.
 constexpr int kMaxDevices = 64;
-std::atomic<uint8_t> g_lds_ready[kMaxDevices][kNumTiles][2][2][kModes];
+std::atomic<uint8_t> g_lds_ready[kMaxDevices][kNumTiles + 1][2][2][kModes];
 
-int ensure_lds_limit(const TileConfig* tile, int packed, int acc, int mode) {
-  if (tile->lds <= 65536) return FA_OK;
+// `slot` is the kernel's index in g_lds_ready: its tile's, or kNumTiles for
+// the few-row kernel.
+int ensure_lds_limit(attn_fn fn, int lds, int slot, int packed, int acc, int mode) {
+  if (lds <= 65536) return FA_OK;
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return FA_ERR_LAUNCH;
-  std::atomic<uint8_t>& ready = g_lds_ready[dev][tile - kTiles][packed][acc][mode];
+  std::atomic<uint8_t>& ready = g_lds_ready[dev][slot][packed][acc][mode];
   if (ready.load(std::memory_order_acquire)) return FA_OK;
-  if (hipFuncSetAttribute(reinterpret_cast<const void*>(tile->fn[packed][acc][mode]),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, tile->lds) != hipSuccess)
+  if (hipFuncSetAttribute(reinterpret_cast<const void*>(fn),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
     return FA_ERR_LAUNCH;
   ready.store(1, std::memory_order_release);
   return FA_OK;
@@ -1775,7 +2138,10 @@ int launch(const fa_problem* p, const fa_strides* strides, const void* q, const 
   const int packed = row_layout(p).pack > 1 ? 1 : 0;
   rc = check_stream_device(stream);
   if (rc) return rc;
-  rc = ensure_lds_limit(tile, packed, acc, mode);
+  const bool rows_kernel = mode == MODE_SPLIT && few_rows(p, splits);
+  const attn_fn fn = rows_kernel ? kRowsFn[packed][acc] : tile->fn[packed][acc][mode];
+  const int lds = rows_kernel ? kRowsLds : tile->lds;
+  rc = ensure_lds_limit(fn, lds, rows_kernel ? kNumTiles : (int)(tile - kTiles), packed, acc, mode);
   if (rc) return rc;
   if (!cus) {
     rc = device_cus(&cus);
@@ -1816,7 +2182,7 @@ int launch(const fa_problem* p, const fa_strides* strides, const void* q, const 
     // The natural-V tile without copies needs the pad kernel only for
     // the counter, which a launch of at most one work item per CU does not
     // use (fa_pp_body): then nothing runs before the attention kernel.
-    const bool direct = grid_size(p) * splits <= (uint64_t)cus;
+    const bool direct = rows_kernel || grid_size(p) * splits <= (uint64_t)cus;
     bool ok = true;
     if (!lay.vnat)
       ok = hipLaunchKernel(reinterpret_cast<const void*>(&fa_prep_kernel), groups, dim3(256),
@@ -1838,7 +2204,7 @@ int launch(const fa_problem* p, const fa_strides* strides, const void* q, const 
   args.opart = reinterpret_cast<float*>(static_cast<char*>(workspace) + sl.opart_offset);
   args.lpart = reinterpret_cast<float*>(static_cast<char*>(workspace) + sl.lpart_offset);
   args.next_tile = next_tile;
-  args.tiles = (int)grid_size(p);
+  args.tiles = (int)(rows_kernel ? row_tiles(p) : grid_size(p));
   args.splits = splits;
   args.heads_q = (int)p->heads_q;
   args.group = (int)(p->heads_q / p->heads_kv);
@@ -1855,9 +2221,14 @@ int launch(const fa_problem* p, const fa_strides* strides, const void* q, const 
   void* attn_args[] = {&args};
   // One workgroup per CU (the LDS ring leaves room for no second one), never
   // more workgroups than work items.
-  const unsigned grid = (unsigned)std::min<uint64_t>(grid_size(p) * splits, (uint64_t)cus);
-  if (hipLaunchKernel(reinterpret_cast<const void*>(tile->fn[packed][acc][mode]), dim3(grid),
-                      dim3(kThreads), attn_args, tile->lds, st) != hipSuccess)
+  // The few-row kernel has one workgroup per item, the (KV head, part) units
+  // rounded up to whole rounds over the 8 dies (see its index map).
+  const uint64_t kv_heads = (uint64_t)(p->batch * p->heads_kv);
+  const unsigned grid =
+      rows_kernel ? (unsigned)((kv_heads * splits + 7) / 8 * 8 * (args.tiles / kv_heads))
+                  : (unsigned)std::min<uint64_t>(grid_size(p) * splits, (uint64_t)cus);
+  if (hipLaunchKernel(reinterpret_cast<const void*>(fn), dim3(grid), dim3(kThreads), attn_args, lds,
+                      st) != hipSuccess)
     return FA_ERR_LAUNCH;
   if (splits > 1) {
     const float* opart = args.opart;
