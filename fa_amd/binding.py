@@ -155,6 +155,9 @@ class AttentionConfig:
                 raise ValueError("the key-split forward has no capture, trace or sync mode")
 
 
+LAYOUT_ERROR = ("Q/K/V must be [B,H,N,128] views with a contiguous last dimension and 16-byte "
+                "aligned rows")
+
 # Query rows per attention tile.
 TILE_ROWS = 256
 
@@ -183,6 +186,15 @@ def make_problem(q_shape, k_shape, scale, config):
                      FA_CAUSAL[config.causal])
 
 
+class Plan:
+    """What a call derives from its signature alone (shapes, strides, dtypes,
+    devices, scale and outputs): the checks of ``Operator.validate`` passed,
+    the problem and the library function with the arguments around the
+    pointers, the output buffers and the workspace size."""
+    __slots__ = ("config", "fn", "before", "after", "size", "out", "lse", "stats", "block", "trace",
+                 "outputs", "extra")
+
+
 class Operator:
     """Callable ``(q, k, v) -> o`` over ``libfa_hip.so``."""
 
@@ -191,7 +203,8 @@ class Operator:
         self.lib = load_library(library) if not isinstance(library, C.CDLL) else library
         self.workspace = None
         self.buffers = {}
-        self.plans = {}          # (shapes, scale, device) -> (FaProblem, workspace bytes)
+        self.plans = {}          # call signature -> Plan
+        self.streams = {}        # (device index, raw stream) -> torch stream
         self.tiles = {}          # (q shape, k shape) -> (rows, keys) granularity
         self.last = None
 
@@ -252,8 +265,7 @@ class Operator:
             st = t.stride()
             if st[3] != 1 or any(x % 8 or x < 0 for x in st[:3]) or st[2] < 128 \
                     or t.data_ptr() % 16:
-                raise ValueError("Q/K/V must be [B,H,N,128] views with a contiguous last "
-                                 "dimension and 16-byte aligned rows")
+                raise ValueError(LAYOUT_ERROR)
 
     def buffers_for(self, q, k, lse=False):
         import torch
@@ -309,73 +321,103 @@ class Operator:
         [tiles, 8]: the per-query-tile records of ``fa_fwd_trace``."""
         import torch
 
+        # Everything but the pointers' alignment follows from these values,
+        # so one lookup stands for the checks and the set-up of a signature
+        # met before: a call's host time is 12 us of which the launches are 6
+        # (24 us with every check and conversion made anew), which is what
+        # bounds a short decode step.
+        if scale is not None:
+            scale = float(scale)
+        key = (q.shape, k.shape, v.shape, q.stride(), k.stride(), v.stride(), q.dtype, k.dtype,
+               v.dtype, q.device, k.device, v.device, scale, bool(return_lse))
+        plan = self.plans.get(key)
+        if plan is None or plan.config is not self.config:
+            plan = self.plans[key] = self.plan(q, k, v, scale, return_lse)
+        qp, kp, vp = q.data_ptr(), k.data_ptr(), v.data_ptr()
+        if (qp | kp | vp) % 16:
+            raise ValueError(LAYOUT_ERROR)
+        index = q.device.index
+        if index == torch.cuda.current_device():
+            self.launch(plan, q, k, v, qp, kp, vp, index)
+        else:
+            with torch.cuda.device(index):
+                self.launch(plan, q, k, v, qp, kp, vp, index)
+        self.last = {"output": plan.out, "lse": plan.lse, "stats": plan.stats,
+                     "block_keys": plan.block, "trace": plan.trace}
+        return (plan.out, plan.lse) if return_lse else plan.out
+
+    def plan(self, q, k, v, scale, return_lse):
+        """The Plan of a call signature; raises what the call must refuse."""
+        import torch
+
         self.validate(q, k, v)
-        scale = q.shape[3] ** -0.5 if scale is None else float(scale)
+        scale = q.shape[3] ** -0.5 if scale is None else scale
         if not (scale > 0 and math.isfinite(scale)):
             raise ValueError("scale must be finite and positive")
-        splits = self.config.splits
-        # The problem and its workspace size depend on the shapes, the scale
-        # and (automatic split count) the device only: computed once each.
-        plan_key = (tuple(q.shape), tuple(k.shape), scale, q.device)
-        if plan_key not in self.plans:
-            prob = make_problem(q.shape, k.shape, scale, self.config)
-            size = C.c_uint64()
-            if splits is None:
-                self.check(self.lib.fa_fwd_workspace_bytes(C.byref(prob), C.byref(size)),
-                           "prepare")
-            else:
-                with torch.cuda.device(q.device):
-                    self.check(self.lib.fa_fwd_split_workspace_bytes(C.byref(prob), splits,
-                                                                     C.byref(size)), "prepare")
-            self.plans[plan_key] = (prob, size.value)
-        prob, size = self.plans[plan_key]
-        out = self.buffers_for(q, k)
-        capture = self.config.capture
-        lse = self.buffers_for(q, k, lse=True) if (return_lse or capture) else None
-        stats, block = self.stats_for(q, k, prob) if capture else (None, 0)
-        trace = self.trace_for(q, k, prob) if self.config.trace else None
+        config, splits, lib = self.config, self.config.splits, self.lib
+        prob = make_problem(q.shape, k.shape, scale, config)
+        size = C.c_uint64()
+        if splits is None:
+            self.check(lib.fa_fwd_workspace_bytes(C.byref(prob), C.byref(size)), "prepare")
+        else:
+            with torch.cuda.device(q.device):
+                self.check(lib.fa_fwd_split_workspace_bytes(C.byref(prob), splits,
+                                                            C.byref(size)), "prepare")
+        p = Plan()
+        p.config, p.size = config, max(size.value, 16)
+        p.out = self.buffers_for(q, k)
+        capture = config.capture
+        p.lse = self.buffers_for(q, k, lse=True) if (return_lse or capture) else None
+        p.stats, p.block = self.stats_for(q, k, prob) if capture else (None, 0)
+        p.trace = self.trace_for(q, k, prob) if config.trace else None
         strided = not all(t.is_contiguous() for t in (q, k, v))
-        if strided and (capture or trace is not None or self.config.sync):
+        if strided and (capture or p.trace is not None or config.sync):
             raise ValueError("capture, trace and sync modes need contiguous Q/K/V")
-        with torch.cuda.device(q.device):
-            need = max(size, 16)
-            if self.workspace is None or self.workspace.device != q.device \
-                    or self.workspace.numel() < need:
-                self.workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
-            stream = torch.cuda.current_stream(q.device)
-            common = (q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr())
-            tail = (self.workspace.data_ptr(), self.workspace.numel(),
-                    C.c_void_p(stream.cuda_stream))
-            st = None
-            if strided:
-                st = FaStrides()
-                for name, t in (("q", q), ("k", k), ("v", v), ("o", out)):
-                    getattr(st, name)[:] = t.stride()[:3]
-            if splits is not None:
-                status = self.lib.fa_fwd_split(C.byref(prob), splits,
-                                               C.byref(st) if st is not None else None, *common,
-                                               lse.data_ptr() if lse is not None else None, *tail)
-            elif strided:
-                status = self.lib.fa_fwd_strided(C.byref(prob), C.byref(st), *common,
-                                                 lse.data_ptr() if lse is not None else None,
-                                                 *tail)
-            elif capture:
-                status = self.lib.fa_fwd_capture(C.byref(prob), *common, lse.data_ptr(),
-                                                 stats.data_ptr(), stats.numel(), *tail)
-            elif trace is not None:
-                status = self.lib.fa_fwd_trace(C.byref(prob), *common, trace.data_ptr(),
-                                               trace.numel(), *tail)
-            elif self.config.sync:
-                status = self.lib.fa_fwd_sync(C.byref(prob), *common,
-                                              lse.data_ptr() if lse is not None else None, *tail)
-            elif return_lse:
-                status = self.lib.fa_fwd_lse(C.byref(prob), *common, lse.data_ptr(), *tail)
-            else:
-                status = self.lib.fa_fwd(C.byref(prob), *common, *tail)
+        st = None
+        if strided:
+            st = FaStrides()
+            for name, t in (("q", q), ("k", k), ("v", v), ("o", p.out)):
+                getattr(st, name)[:] = t.stride()[:3]
+            st = C.byref(st)
+        # The call is fn(*before, q, k, v, *outputs, *after, workspace, bytes, stream);
+        # an output of None is passed as a null pointer.
+        p.before, p.outputs, p.after = (C.byref(prob),), (p.out, p.lse), ()
+        if splits is not None:
+            p.fn, p.before = lib.fa_fwd_split, (C.byref(prob), splits, st)
+        elif strided:
+            p.fn, p.before = lib.fa_fwd_strided, (C.byref(prob), st)
+        elif capture:
+            p.fn, p.outputs = lib.fa_fwd_capture, (p.out, p.lse, p.stats)
+            p.after = (p.stats.numel(),)
+        elif p.trace is not None:
+            p.fn, p.outputs, p.after = lib.fa_fwd_trace, (p.out, p.trace), (p.trace.numel(),)
+        elif config.sync:
+            p.fn = lib.fa_fwd_sync
+        elif return_lse:
+            p.fn = lib.fa_fwd_lse
+        else:
+            p.fn, p.outputs = lib.fa_fwd, (p.out,)
+        p.extra = tuple(t for t in (p.out, p.lse, p.stats, p.trace) if t is not None)
+        return p
+
+    def launch(self, plan, q, k, v, qp, kp, vp, index):
+        """Enqueue the planned call on the current stream of device `index`,
+        which is the current device."""
+        import torch
+
+        ws = self.workspace
+        if ws is None or ws.device != q.device or ws.numel() < plan.size:
+            ws = self.workspace = torch.empty(plan.size, dtype=torch.uint8, device=q.device)
+        raw = torch._C._cuda_getCurrentRawStream(index)
+        stream = self.streams.get((index, raw))
+        if stream is None:
+            if len(self.streams) >= 64:
+                self.streams.clear()
+            stream = self.streams[index, raw] = torch.cuda.current_stream(index)
+        outputs = [t.data_ptr() if t is not None else None for t in plan.outputs]
+        status = plan.fn(*plan.before, qp, kp, vp, *outputs, *plan.after, ws.data_ptr(), ws.numel(),
+                         raw)
+        if status:
             self.check(status, "launch")
-            extra = tuple(t for t in (lse, stats, trace) if t is not None)
-            for t in (q, k, v, out, self.workspace) + extra:
-                t.record_stream(stream)
-        self.last = {"output": out, "lse": lse, "stats": stats, "block_keys": block,
-                     "trace": trace}
-        return (out, lse) if return_lse else out
+        for t in (q, k, v, ws) + plan.extra:
+            t.record_stream(stream)
