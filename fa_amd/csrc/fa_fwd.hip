@@ -1851,17 +1851,19 @@ SplitLayout split_layout(const fa_problem* p, const KeyLayout& lay, int splits) 
 // Largest accepted split count (fa_fwd_split's splits argument).
 constexpr int kMaxSplits = 1024;
 // Split counts the automatic choice considers: every count up to
-// kAutoSplitMax without a mask (the model is a closed form there), these
-// with a causal mask (the model sums over the tiles).
+// kAutoSplitMax without a mask (the model is a closed form there); with a
+// causal mask (the model sums over the tiles) only those of at most
+// kAutoCausalItems work items per CU, but at least up to 16.
 constexpr int kAutoSplitMax = 256;
-constexpr int kAutoSplitsCausal[] = {2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64, 96, 128, 192, 256};
+constexpr int kAutoCausalItems = 8;
 
 // Modelled duration of a launch whose tiles' key ranges are cut into s
 // parts, in units of one key block's time on one workgroup. A work item
 // costs its key blocks plus kItemOverhead (pipeline fill and drain,
 // epilogue), an empty item (a causal part past the diagonal) almost nothing.
-// Equal items (full attention) run in ceil(items / cus) rounds; unequal ones
-// (causal) are bounded by max(total / cus, longest item), which the work
+// Equal items (full attention) run in ceil(items / cus) rounds; with a causal
+// mask the parts a tile sees whole do, and all items are bounded by
+// max(total / cus, longest item), which the work
 // queue, handing out the longest tiles first, comes close to. A split launch
 // adds the merge kernel: it reads every part's O and lse and writes O, at
 // kMergeBytesPerSecond, but no faster than one row's walk over its parts
@@ -1888,20 +1890,19 @@ double split_cost(const fa_problem* p, const TileConfig* tile, const KeyLayout& 
     t = ceil(items / cus) * per;
   } else {
     const int64_t off = p->causal == FA_CAUSAL_BOTTOM_RIGHT ? p->seq_k - p->seq_q : 0;
-    double total = 0.0, longest = 0.0;
+    const int64_t len = (nbt + s - 1) / s;                 // longest part
+    double total = 0.0, longest = 0.0, whole = 0.0;
     for (int64_t r = 0; r < tiles_q; ++r) {
-      // Keys [0, kend) are seen by the tile's last row (its position + 1).
+      // Keys [0, kend) are seen by the tile's last row (its position + 1):
+      // vis key blocks, which fill some parts and reach into one more.
       const int64_t kend = (std::min<int64_t>((r + 1) * kRows, rl.rows) - 1) / rl.pack + 1 + off;
       const int64_t vis = kend <= 0 ? 0 : std::min<int64_t>(nbt, (kend + bn - 1) / bn);
-      for (int i = 0; i < s; ++i) {
-        const int64_t b0 = i * nbt / s, b1 = (i + 1) * nbt / s;
-        const int64_t nb = std::max<int64_t>(0, std::min(vis, b1) - b0);
-        const double cost = nb > 0 ? nb + kItemOverhead : kEmptyItem;
-        total += cost * nbh;
-        longest = std::max(longest, cost);
-      }
+      const int64_t seen = (vis * s + nbt - 1) / nbt;
+      total += (double)nbh * (vis + seen * kItemOverhead + (s - seen) * kEmptyItem);
+      longest = std::max(longest, std::min(vis, len) + kItemOverhead);
+      whole += (double)(nbh * ((2 * vis * s + nbt - 1) / (2 * nbt)));   // parts seen by more than half
     }
-    t = std::max(total / cus, longest);
+    t = std::max({total / cus, longest, ceil(whole / cus) * (nbt / s + kItemOverhead)});
   }
   if (s > 1) {
     const double rows = (double)(p->batch * p->heads_q) * p->seq_q;
@@ -1978,11 +1979,11 @@ int resolve_splits(const fa_problem* p, const TileConfig* tile, const KeyLayout&
           s = c;
         }
       };
-      if (p->causal == FA_CAUSAL_NONE) {
-        for (int c = 2; c <= kAutoSplitMax; ++c) consider(c);
-      } else {
-        for (int c : kAutoSplitsCausal) consider(c);
-      }
+      int most = kAutoSplitMax;
+      if (p->causal != FA_CAUSAL_NONE)
+        most = (int)std::min<int64_t>(
+            most, std::max<int64_t>(16, kAutoCausalItems * cus / (int64_t)grid_size(p)));
+      for (int c = 2; c <= most; ++c) consider(c);
     }
   }
   if ((int64_t)grid_size(p) * s >= ((int64_t)1 << 30)) return FA_ERR_GEOMETRY;
