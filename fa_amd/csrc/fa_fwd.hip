@@ -604,6 +604,7 @@ __device__ __forceinline__ void fa_pp_tile(const FaArgs& args, const int tile, c
   static_assert(KBYTES == KI * 1024 && VBYTES == VI * 1024, "blocks are whole DMA instructions");
   constexpr int PF = 4;                  // LDS operand prefetch depth (MFMAs)
   constexpr float TAU = ACC16 ? 0.f : 8.f;
+  constexpr int BOTH = 0, QK = 1, PV = 2;   // what an MFMA step computes
 
   extern __shared__ __attribute__((aligned(16))) char lds[];
   char* kbase = lds;                     // NS K blocks
@@ -819,9 +820,11 @@ __device__ __forceinline__ void fa_pp_tile(const FaArgs& args, const int tile, c
     __builtin_amdgcn_sched_barrier(0);
   };
   static_assert((NS - 2) * NIW <= 24 && NS >= 2, "wait_dma covers at most 24 loads");
-  // MFMA index after which DMA instruction m is issued inside an MFMA step.
-  constexpr int DSTEP = (2 * NQK - 8) / NIW > 0 ? (2 * NQK - 8) / NIW : 1;
-  static_assert(1 + DSTEP * (NIW - 1) < 2 * NQK, "every DMA instruction finds an MFMA slot");
+  // MFMAs between the DMA instructions of an MFMA step of n MFMAs, the first
+  // of which goes out after MFMA 1.
+  auto dma_step = [](int n) constexpr { return (n - 8) / NIW > 0 ? (n - 8) / NIW : 1; };
+  static_assert(1 + dma_step(NQK) * (NIW - 1) < NQK && 1 + dma_step(2 * NQK) * (NIW - 1) < 2 * NQK,
+                "every DMA instruction finds an MFMA slot");
   static_assert(NIW <= 8 * KT, "every DMA instruction finds an exponential pair of a VALU step");
 
   f32x16 acc[4];
@@ -848,8 +851,6 @@ __device__ __forceinline__ void fa_pp_tile(const FaArgs& args, const int tile, c
         acc[dt][i + 1] = (float)t[1];
       }
   };
-#pragma unroll
-  for (int i = 0; i < KS; ++i) p[i] = h8{};
 
   // Per-lane operand offsets. QK op (t, kk) reads K row 32t + l32, chunk
   // 2kk + hf. PV op (dt, ks) needs, for dim 32dt + l32, the keys 16ks + 4hf
@@ -871,7 +872,12 @@ __device__ __forceinline__ void fa_pp_tile(const FaArgs& args, const int tile, c
   }
 
   // MFMA step for block j: S^T(j) = K(j) Q^T and O^T += V^T(j-1) P^T(j-1),
-  // QK and PV MFMAs interleaved, operands prefetched PF MFMAs ahead.
+  // QK and PV MFMAs interleaved, operands prefetched PF MFMAs ahead. The first
+  // step of a tile has only the QK half, the one after its last block only
+  // the PV half (KIND; with both halves in each, a tile's MFMAs took two half
+  // steps on each group more: a batch of 4 x 32 heads over 2048 keys, 2 to 16
+  // blocks a tile, 182 us instead of 180; 1000 causal rows, 8 blocks, 31.4
+  // instead of 30.0; 256 blocks a tile 2 % more).
   // Operand i of a step: QK op n = i / 2 (even i) covers S tile n % KT at
   // k-step n / KT, so consecutive QK ops alternate accumulators; with PV ops
   // in between, no accumulator is reused within four MFMAs and dependent
@@ -896,25 +902,30 @@ __device__ __forceinline__ void fa_pp_tile(const FaArgs& args, const int tile, c
   // earlier), so its MFMA step starts without waiting for LDS; a group-0
   // step reads them itself.
   h8 fr[PF];
-  auto preload = [&](const char* kb, const char* vb) {
+  // Operand of MFMA i of a step of the given kind.
+  auto operand = [](int kind, int i) constexpr { return kind == BOTH ? i : 2 * i + (kind == PV); };
+  auto preload = [&](const char* kb, const char* vb, auto kind) {
 #pragma unroll
-    for (int i = 0; i < PF; ++i) fr[i] = ld(kb, vb, i);
+    for (int i = 0; i < PF; ++i) fr[i] = ld(kb, vb, operand(decltype(kind)::value, i));
   };
   auto mfma_step = [&](const char* kb, const char* vb, bool with_dma, int dkb, int dks, int dvb,
-                       int dvs, auto preloaded) {
-    if constexpr (!decltype(preloaded)::value) preload(kb, vb);
+                       int dvs, auto preloaded, auto kind) {
+    constexpr int KIND = decltype(kind)::value;
+    constexpr int N = KIND == BOTH ? 2 * NQK : NQK;
+    constexpr int DSTEP = dma_step(N);
+    if constexpr (!decltype(preloaded)::value) preload(kb, vb, kind);
 #pragma unroll
-    for (int i = 0; i < 2 * NQK; ++i) {
+    for (int i = 0; i < N; ++i) {
       const h8 a = fr[i % PF];
-      const int n = i >> 1;
+      const int op = operand(KIND, i), n = op >> 1;
       // The first product into each S tile starts from a zero accumulator
       // operand instead of zeroed registers.
-      if ((i & 1) == 0) {
+      if ((op & 1) == 0) {
         s[n % KT] = mfma32(a, qf[n / KT], n < KT ? f32x16{} : s[n % KT]);
       } else {
         acc[n % 4] = mfma32(a, p[n / 4], acc[n % 4]);
       }
-      if (i + PF < 2 * NQK) fr[i % PF] = ld(kb, vb, i + PF);
+      if (i + PF < N) fr[i % PF] = ld(kb, vb, operand(KIND, i + PF));
       if (i >= 1 && (i - 1) % DSTEP == 0 && (i - 1) / DSTEP < NIW) {
         if (with_dma) dma_one((i - 1) / DSTEP, dkb, dks, dvb, dvs);
       }
@@ -930,11 +941,6 @@ __device__ __forceinline__ void fa_pp_tile(const FaArgs& args, const int tile, c
       reinterpret_cast<u32x4*>(lds)[i] = u32x4{NAN16X2, NAN16X2, NAN16X2, NAN16X2};
     lds_barrier();
   }
-  // V slot NS-1 (read as "V(-1)" by the first MFMA step) starts as zeros:
-  // the first step multiplies it by P = 0.
-  for (int i = tid; i < VBYTES / 16; i += NT)
-    reinterpret_cast<u32x4*>(vbase + (NS - 1) * VBYTES)[i] = u32x4{0u, 0u, 0u, 0u};
-
   const int last = nblk - 1;
   // Prologue (group 0): K(0..NS-2) -> slots 0..NS-2 and V(0..NS-3) -> slots
   // 0..NS-3, everything pairs before pair 0 would have loaded. Block indices
@@ -1074,6 +1080,9 @@ __device__ __forceinline__ void fa_pp_tile(const FaArgs& args, const int tile, c
   // slower than no test, even when never taken.
   const std::integral_constant<bool, false> unmasked, loads;
   const std::integral_constant<bool, true> masked, preloaded;
+  const std::integral_constant<int, BOTH> both;
+  const std::integral_constant<int, QK> qk;
+  const std::integral_constant<int, PV> pv;
   const int nfull = klim_w + 1 < BN ? 0 : min(nblk, (klim_w + 1) / BN);
   int sl = 0;
   // Who issues the loads. Pair t's loads, K(t+NS-1) -> slot (t-1) % NS and
@@ -1128,21 +1137,34 @@ __device__ __forceinline__ void fa_pp_tile(const FaArgs& args, const int tile, c
       lds_barrier();                           // phase 2 nblk + 1
     }
   } else if (grp == 0) {
-    auto pair = [&](int j, auto mask) {
+    auto mfma = [&](int j, auto kind) {        // phase 2j: pair j starts
       const int sp = prev(sl);
       mfma_step(kslot(sl), vslot(sp), !LOADS_IN_VALU, min(j + NS - 1, last), sp,
-                min(j + NS - 2, last), prev(sp), loads);   // phase 2j: pair j starts
+                min(j + NS - 2, last), prev(sp), loads, kind);
       if constexpr (SYNC && !LOADS_IN_VALU) wait_dma(0);   // sync mode: loads land in their phase
       lds_barrier();
-      valu_step(j * BN, mask, [](int) {});   // phase 2j + 1
+    };
+    auto valu = [&](int j, auto mask) {        // phase 2j + 1
+      valu_step(j * BN, mask, [](int) {});
       if constexpr (!LOADS_IN_VALU) wait_dma(keep);        // K(j+1), V(j) have landed
       lds_barrier();
       sl = next(sl);
     };
-    int j = 0;
-    for (; j < nfull; ++j) pair(j, unmasked);
-    for (; j < nblk; ++j) pair(j, masked);
-    mfma_step(kslot(sl), vslot(prev(sl)), false, 0, 0, 0, 0, loads);   // phase 2 nblk: PV(nblk - 1)
+    mfma(0, qk);
+    if (nfull > 0)
+      valu(0, unmasked);
+    else
+      valu(0, masked);
+    int j = 1;
+    for (; j < nfull; ++j) {
+      mfma(j, both);
+      valu(j, unmasked);
+    }
+    for (; j < nblk; ++j) {
+      mfma(j, both);
+      valu(j, masked);
+    }
+    mfma_step(kslot(sl), vslot(prev(sl)), false, 0, 0, 0, 0, loads, pv);   // phase 2 nblk: PV(nblk - 1)
     lds_barrier();
     lds_barrier();                           // phase 2 nblk + 1: idle
   } else {
@@ -1150,12 +1172,14 @@ __device__ __forceinline__ void fa_pp_tile(const FaArgs& args, const int tile, c
       issue(min(NS - 1, last), NS - 1, min(NS - 2, last), NS - 2);
       if constexpr (SYNC) wait_dma(0);
     }
-    preload(kslot(0), vslot(NS - 1));  // phase 0: this group idles
+    preload(kslot(0), vslot(0), qk);   // phase 0: this group idles
     lds_barrier();
-    auto pair = [&](int j, auto mask) {
-      mfma_step(kslot(sl), vslot(prev(sl)), false, 0, 0, 0, 0, preloaded);   // phase 2j + 1
+    auto mfma = [&](auto kind) {         // phase 2j + 1
+      mfma_step(kslot(sl), vslot(prev(sl)), false, 0, 0, 0, 0, preloaded, kind);
       if constexpr (LOADS_IN_VALU) wait_dma(keep);         // K(j+1), V(j) have landed
       lds_barrier();
+    };
+    auto valu = [&](int j, auto mask) {  // phase 2j + 2
       // Pair j + 1's loads, K(j+NS) -> slot sl and V(j+NS-1) -> prev(sl),
       // spread over the step's exponentials (in a burst at its start they
       // measured slower and fetched 4x the bytes from beyond L2).
@@ -1170,18 +1194,29 @@ __device__ __forceinline__ void fa_pp_tile(const FaArgs& args, const int tile, c
               __builtin_amdgcn_sched_barrier(0);
             }
         }
-      });                            // phase 2j + 2
+      });
       if constexpr (LOADS_IN_VALU && SYNC) wait_dma(0);
       // K(j+1) and V(j), the next step's blocks, were published at this
       // phase's barrier, and no load writes their slots before pair j + 2.
-      preload(kslot(next(sl)), vslot(sl));
+      preload(kslot(next(sl)), vslot(sl), both);
       lds_barrier();
       sl = next(sl);
     };
-    int j = 0;
-    for (; j < nfull; ++j) pair(j, unmasked);
-    for (; j < nblk; ++j) pair(j, masked);
-    mfma_step(kslot(sl), vslot(prev(sl)), false, 0, 0, 0, 0, preloaded);   // phase 2 nblk + 1: PV(nblk - 1)
+    mfma(qk);
+    if (nfull > 0)
+      valu(0, unmasked);
+    else
+      valu(0, masked);
+    int j = 1;
+    for (; j < nfull; ++j) {
+      mfma(both);
+      valu(j, unmasked);
+    }
+    for (; j < nblk; ++j) {
+      mfma(both);
+      valu(j, masked);
+    }
+    mfma_step(kslot(sl), vslot(prev(sl)), false, 0, 0, 0, 0, loads, pv);   // phase 2 nblk + 1: PV(nblk - 1)
     lds_barrier();
   }
   // No DMA may still be writing this workgroup's LDS when it exits.
