@@ -781,20 +781,31 @@ __device__ __forceinline__ void fa_pp_tile(const FaArgs& args, const int tile, c
   const i32x4 vrsrc = VNAT ? buffer_rsrc(vp + (size_t)kb0 * BN * args.vs.n, (nk_valid - kb0 * BN - 1) * vrow + HD * 2)
                            : buffer_rsrc(vp + kb0 * BN, seq_k * (HD * 2) - kb0 * (BN * 2));
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
-  // DMA instruction m of this wave for K block kb -> ring slot ks and V
-  // block vb -> slot vs. Branch free: the K/V choice is a select on
-  // wave-uniform values; only a wave's last instruction can be absent.
-  auto dma_one = [&](int m, int kb, int ks, int vb, int vs) {
+  // Byte offsets of K block kb and V block vb in their buffers, or, for a
+  // block past the tile's last one, an offset past any buffer's end: such a
+  // load is issued like any other (which keeps the wait counts fixed) but
+  // fetches nothing. (Loading the last block again in its place cost 1.5
+  // blocks of L2 traffic per tile.)
+  const int last = nblk - 1;
+  constexpr int NOWHERE = 0x7ff00000;
+  auto koff = [&](int kb) { return kb <= last ? kb * (BN * krow) : NOWHERE; };
+  auto voff = [&](int vb) { return vb <= last ? vb * (VNAT ? BN * vrow : BN * 2) : NOWHERE; };
+  // DMA instruction m of this wave for the K block at offset ko -> ring slot
+  // ks and the V block at offset vo -> slot vs. Branch free: the K/V choice is
+  // a select on wave-uniform values; only a wave's last instruction can be
+  // absent.
+  auto dma_one = [&](int m, int ko, int ks, int vo, int vs) {
     const int q = dw + 4 * m;
     if (m == NIW - 1 && NI % 4 != 0 && q >= NI) return;
     const bool isk = q < KI;
     const int dst = isk ? ks * KBYTES + q * 1024 : NS * KBYTES + vs * VBYTES + (q - KI) * 1024;
-    const int soff = isk ? kb * (BN * krow) : VNAT ? (vb * BN + 4 * (q - KI)) * vrow : vb * (BN * 2);
+    const int soff = isk ? ko : VNAT ? vo + 4 * (q - KI) * vrow : vo;
     dma_to_lds(isk ? krsrc : vrsrc, lds0 + dst, m < NOFF ? dma_off[m] : vdma, soff);
   };
   auto issue = [&](int kb, int ks, int vb, int vs) {
+    const int ko = koff(kb), vo = voff(vb);
 #pragma unroll
-    for (int m = 0; m < NIW; ++m) dma_one(m, kb, ks, vb, vs);
+    for (int m = 0; m < NIW; ++m) dma_one(m, ko, ks, vo, vs);
   };
   // Wait until at most n of this wave's DMA loads are outstanding.
   auto wait_dma = [&](int n) {
@@ -917,7 +928,7 @@ __device__ __forceinline__ void fa_pp_tile(const FaArgs& args, const int tile, c
 #pragma unroll
     for (int i = 0; i < PF; ++i) fr[i] = ld(kb, vb, operand(decltype(kind)::value, i));
   };
-  auto mfma_step = [&](const char* kb, const char* vb, bool with_dma, int dkb, int dks, int dvb,
+  auto mfma_step = [&](const char* kb, const char* vb, bool with_dma, int dko, int dks, int dvo,
                        int dvs, auto preloaded, auto kind) {
     constexpr int KIND = decltype(kind)::value;
     constexpr int N = KIND == BOTH ? 2 * NQK : NQK;
@@ -936,7 +947,7 @@ __device__ __forceinline__ void fa_pp_tile(const FaArgs& args, const int tile, c
       }
       if (i + PF < N) fr[i % PF] = ld(kb, vb, operand(KIND, i + PF));
       if (i >= 1 && (i - 1) % DSTEP == 0 && (i - 1) / DSTEP < NIW) {
-        if (with_dma) dma_one((i - 1) / DSTEP, dkb, dks, dvb, dvs);
+        if (with_dma) dma_one((i - 1) / DSTEP, dko, dks, dvo, dvs);
       }
       // Keep source order: operand reads stay PF MFMAs ahead of their use.
       __builtin_amdgcn_sched_barrier(0);
@@ -950,16 +961,13 @@ __device__ __forceinline__ void fa_pp_tile(const FaArgs& args, const int tile, c
       reinterpret_cast<u32x4*>(lds)[i] = u32x4{NAN16X2, NAN16X2, NAN16X2, NAN16X2};
     lds_barrier();
   }
-  const int last = nblk - 1;
   // Prologue (group 0): K(0..NS-2) -> slots 0..NS-2 and V(0..NS-3) -> slots
-  // 0..NS-3, everything pairs before pair 0 would have loaded. Block indices
-  // past the end are clamped, so every pair issues the same loads and the
-  // fixed wait counts stay exact. (issue() always loads one K and one V
+  // 0..NS-3, everything pairs before pair 0 would have loaded. (issue() always loads one K and one V
   // block; the prologue's extra V loads target slots that are rewritten
   // before use.)
   if (grp == 0) {
 #pragma unroll
-    for (int i = 0; i + 1 < NS; ++i) issue(min(i, last), i, min(i, last), i);
+    for (int i = 0; i + 1 < NS; ++i) issue(i, i, i, i);
   }
   wait_dma(0);
   // Every load of this wave has landed, the Q fragments included. Consuming
@@ -1117,7 +1125,7 @@ __device__ __forceinline__ void fa_pp_tile(const FaArgs& args, const int tile, c
       for (int j = 0; j < nblk; ++j) {
         const int sp = prev(sl);
         if constexpr (!LOADS_IN_VALU) {           // phase 2j: pair j's loads
-          issue(min(j + NS - 1, last), sp, min(j + NS - 2, last), prev(sp));
+          issue(j + NS - 1, sp, j + NS - 2, prev(sp));
           if constexpr (SYNC) wait_dma(0);
         }
         lds_barrier();
@@ -1126,10 +1134,11 @@ __device__ __forceinline__ void fa_pp_tile(const FaArgs& args, const int tile, c
         sl = next(sl);
       }
       lds_barrier();                           // phase 2 nblk
+      wait_dma(0);
       lds_barrier();                           // phase 2 nblk + 1
     } else {
       if constexpr (LOADS_IN_VALU) {           // phase 0: pair 0's loads
-        issue(min(NS - 1, last), NS - 1, min(NS - 2, last), NS - 2);
+        issue(NS - 1, NS - 1, NS - 2, NS - 2);
         if constexpr (SYNC) wait_dma(0);
       }
       lds_barrier();
@@ -1137,19 +1146,20 @@ __device__ __forceinline__ void fa_pp_tile(const FaArgs& args, const int tile, c
         if constexpr (LOADS_IN_VALU) wait_dma(keep);   // phase 2j + 1
         lds_barrier();
         if constexpr (LOADS_IN_VALU) {         // phase 2j + 2: pair j + 1's loads
-          issue(min(j + NS, last), sl, min(j + NS - 1, last), prev(sl));
+          issue(j + NS, sl, j + NS - 1, prev(sl));
           if constexpr (SYNC) wait_dma(0);
         }
         lds_barrier();
         sl = next(sl);
       }
+      wait_dma(0);
       lds_barrier();                           // phase 2 nblk + 1
     }
   } else if (grp == 0) {
     auto mfma = [&](int j, auto kind) {        // phase 2j: pair j starts
       const int sp = prev(sl);
-      mfma_step(kslot(sl), vslot(sp), !LOADS_IN_VALU, min(j + NS - 1, last), sp,
-                min(j + NS - 2, last), prev(sp), loads, kind);
+      mfma_step(kslot(sl), vslot(sp), !LOADS_IN_VALU, koff(j + NS - 1), sp, voff(j + NS - 2), prev(sp),
+                loads, kind);
       if constexpr (SYNC && !LOADS_IN_VALU) wait_dma(0);   // sync mode: loads land in their phase
       lds_barrier();
     };
@@ -1175,10 +1185,11 @@ __device__ __forceinline__ void fa_pp_tile(const FaArgs& args, const int tile, c
     }
     mfma_step(kslot(sl), vslot(prev(sl)), false, 0, 0, 0, 0, loads, pv);   // phase 2 nblk: PV(nblk - 1)
     lds_barrier();
+    wait_dma(0);
     lds_barrier();                           // phase 2 nblk + 1: idle
   } else {
     if constexpr (LOADS_IN_VALU) {       // phase 0: pair 0's loads
-      issue(min(NS - 1, last), NS - 1, min(NS - 2, last), NS - 2);
+      issue(NS - 1, NS - 1, NS - 2, NS - 2);
       if constexpr (SYNC) wait_dma(0);
     }
     preload(kslot(0), vslot(0), qk);   // phase 0: this group idles
@@ -1192,14 +1203,14 @@ __device__ __forceinline__ void fa_pp_tile(const FaArgs& args, const int tile, c
       // Pair j + 1's loads, K(j+NS) -> slot sl and V(j+NS-1) -> prev(sl),
       // spread over the step's exponentials (in a burst at its start they
       // measured slower and fetched 4x the bytes from beyond L2).
-      const int kb = min(j + NS, last), ks = sl, vb = min(j + NS - 1, last), vs = prev(sl);
+      const int ko = koff(j + NS), ks = sl, vo = voff(j + NS - 1), vs = prev(sl);
       valu_step(j * BN, mask, [&](int i) {
         if constexpr (LOADS_IN_VALU) {
 #pragma unroll
           for (int mi = 0; mi < NIW; ++mi)
             if (mi * (8 * KT) / NIW == i) {
               __builtin_amdgcn_sched_barrier(0);
-              dma_one(mi, kb, ks, vb, vs);
+              dma_one(mi, ko, ks, vo, vs);
               __builtin_amdgcn_sched_barrier(0);
             }
         }
@@ -1226,10 +1237,11 @@ __device__ __forceinline__ void fa_pp_tile(const FaArgs& args, const int tile, c
       valu(j, masked);
     }
     mfma_step(kslot(sl), vslot(prev(sl)), false, 0, 0, 0, 0, loads, pv);   // phase 2 nblk + 1: PV(nblk - 1)
+    wait_dma(0);
     lds_barrier();
   }
-  // No DMA may still be writing this workgroup's LDS when it exits.
-  wait_dma(0);
+  // Every wave has waited for its loads before the last barrier, so nothing
+  // writes the ring any more, and nobody reads it.
   claim();
   if constexpr (TRACE) trace_record(args, tile, real0, clk0, nblk, BN);
 
@@ -1255,8 +1267,8 @@ __device__ __forceinline__ void fa_pp_tile(const FaArgs& args, const int tile, c
   // that saw no key (causal mask) has l = 0: O = 0 and lse = -inf.
   const float l = half_sum(lsum);
   const float inv = l > 0.f ? 1.f / l : 0.f;
-  if (!row_ok) return;
   if constexpr (SPLIT) {
+    if (!row_ok) return;
     // This part's O / l in FP32 and its log-sum-exp (-inf, with O = 0, for a
     // row that sees no key of the part).
     if (hf == 0) args.lpart[part] = (__builtin_amdgcn_logf(l) + m * c) * LN2;
@@ -1271,8 +1283,15 @@ __device__ __forceinline__ void fa_pp_tile(const FaArgs& args, const int tile, c
       }
     return;
   }
-  if (args.lse && hf == 0) args.lse[grow] = (__builtin_amdgcn_logf(l) + m * c) * LN2;
-  _Float16* orow = row_at(o, args.os, b, head_of(rowc), pos_of(rowc));
+  if (args.lse && hf == 0 && row_ok) args.lse[grow] = (__builtin_amdgcn_logf(l) + m * c) * LN2;
+  // A lane holds 4 dims here and there of one row; stored like that, a store
+  // instruction touches 32 rows in 16-byte pieces, which left 5.3 us between a
+  // workgroup's tiles (2.8 now; B=4, 32 heads, 2048 causal keys: 172.1 -> 164.7
+  // us with the loads past the last block, see koff; one 1000-key causal
+  // prompt 30.2 -> 27.4). The wave turns its 32 rows around in 8 KiB of the ring, which
+  // nobody reads any more, 16-byte chunk ch of row r at position ch ^ r % 16,
+  // and stores whole rows, 4 to an instruction.
+  char* rows = lds + wave_u * (32 * HD * 2);
 #pragma unroll
   for (int dt = 0; dt < 4; ++dt) {
 #pragma unroll
@@ -1282,8 +1301,17 @@ __device__ __forceinline__ void fa_pp_tile(const FaArgs& args, const int tile, c
       for (int e = 0; e < 4; ++e) {
         out[e] = (_Float16)(acc[dt][4 * g + e] * inv);
       }
-      *reinterpret_cast<h4*>(orow + dt * 32 + 8 * g + 4 * hf) = out;
+      *reinterpret_cast<h4*>(rows + l32 * 256 + (((4 * dt + g) ^ (l32 & 15)) << 4) + hf * 8) = out;
     }
+  }
+  const int64_t obase = (int64_t)b * args.os.b + (int64_t)head_of(rowc) * args.os.h +
+                        (int64_t)pos_of(rowc) * args.os.n;   // this lane's row in o
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int r = 4 * i + (lane >> 4);
+    const u32x4 val = *reinterpret_cast<const u32x4*>(rows + r * 256 + (((lane & 15) ^ (r & 15)) << 4));
+    const int64_t at = (int64_t)(uint32_t)__shfl((int)obase, r) | (int64_t)__shfl((int)(obase >> 32), r) << 32;
+    if (qt * BM + wave_u * 32 + r < seq_r) *reinterpret_cast<u32x4*>(o + at + (lane & 15) * 8) = val;
   }
 }
 
