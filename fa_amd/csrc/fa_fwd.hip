@@ -83,12 +83,13 @@ constexpr float LN2 = 0.6931471805599453f;
 // debug mode: every tile's LDS ring starts poisoned with FP16 NaN and each
 // phase's loads complete before the phase ends, so a read of LDS no load has
 // filled, or a race between the loads and the operand reads, changes the
-// output. Split is the key-split mode: a work item is one query tile and one
-// of `splits` contiguous parts of its key range, and it writes that part's
-// normalised FP32 O and log-sum-exp for a merge kernel to combine. All four
-// are separate kernels.
-enum KernelMode { MODE_RUN = 0, MODE_CAPTURE = 1, MODE_TRACE = 2, MODE_SYNC = 3, MODE_SPLIT = 4 };
+// output. Parts is production with tiles cut into parts of their key range
+// (trace and sync can cut tiles too). All are separate kernels: with the
+// parts' code in the production kernel, short launches, which fetch every
+// instruction for the first time, ran 0.5 to 1.3 % slower.
+enum KernelMode { MODE_RUN = 0, MODE_CAPTURE = 1, MODE_TRACE = 2, MODE_SYNC = 3, MODE_PARTS = 4 };
 constexpr int kModes = 5;
+constexpr bool can_cut(int mode) { return mode != MODE_RUN && mode != MODE_CAPTURE; }
 // FP16 quiet NaN in both halves of a 32-bit word: the poison of sync mode.
 constexpr uint32_t NAN16X2 = 0x7e007e00u;
 
@@ -128,11 +129,15 @@ constexpr int kQueueStride = 8;       // ints
 // (causal_off = 0 aligns the mask top-left, Nk - Nq bottom-right); a row that
 // sees no key gets O = 0 and lse = -inf. qs, ks, vs and os are the element
 // strides of q, of the K and natural-layout V buffers read (the caller's k
-// and v, or their contiguous copies) and of o. In split mode (splits >= 2) the kernel writes,
-// instead of o and lse, each part's O normalised by its own row sum into
-// opart (FP32 [splits][B * Hq * Nq][128]) and the part's natural-log
-// log-sum-exp into lpart (FP32 [splits][B * Hq * Nq]; -inf for a part in
-// which the row sees no key, whose opart row then holds zeros).
+// and v, or their contiguous copies) and of o. Tiles from `whole` on are cut
+// into `splits` contiguous parts of their key range, a work item each, which
+// writes, instead of o and lse, the part's O normalised by its own row sum
+// into opart (FP32 [splits][part_rows][128]) and the part's natural-log
+// log-sum-exp into lpart (FP32 [splits][part_rows]; -inf for a part in
+// which the row sees no key, whose opart row then holds zeros), for a merge
+// kernel to combine. A row's index there is its index in [B * Hq * Nq] if
+// every tile is cut (whole = 0), else its place among the rows of the cut
+// tiles, 256 a tile. `direct`: one workgroup per work item.
 struct Strides {
   int64_t b, h, n;   // batch, head and row strides in elements; the 128 dims are contiguous
 };
@@ -150,10 +155,10 @@ struct FaArgs {
   int causal, causal_off;
   float c;
   Strides qs, ks, os;
-  // Split mode only (after the others, so their argument offsets do not move).
   float* opart;
   float* lpart;
-  int splits;          // key-range parts per tile
+  int64_t part_rows;
+  int whole, splits, direct;
   Strides vs;
 };
 
@@ -358,8 +363,14 @@ __global__ void __launch_bounds__(256) fa_poison_kernel(u32x4* p, uint64_t n16) 
 // each lane accumulates 4 of the 128 dims over all parts, with the weights
 // broadcast from the lane that computed them and the O loads independent of
 // each other (unrolled, so several are in flight). 8 rows per 256-thread
-// block, grid-stride over the rows = B * Hq * Nq; o is written through its
-// strides, lse (may be null) contiguously.
+// block, grid-stride over the rows; o is written through its
+// strides, lse (may be null) contiguously. The rows are those of [B * Hq *
+// Nq] (cut.tiles = 0), or those of the cut tiles of a launch, 256 a tile.
+struct CutTiles {
+  int tiles, whole;     // cut tiles, and the tiles before them
+  int tiles_q, pack;    // tiles per row sequence, query heads per position
+  int seq_r;            // rows per sequence
+};
 __device__ __forceinline__ float max32(float x) {
 #pragma unroll
   for (int m = 16; m >= 1; m >>= 1) x = fmaxf(x, __shfl_xor(x, m, 32));
@@ -375,10 +386,17 @@ __global__ void __launch_bounds__(256) fa_merge_kernel(const float* __restrict__
                                                        _Float16* __restrict__ o,
                                                        float* __restrict__ lse, int splits,
                                                        int64_t rows, int heads_q, int seq_q,
-                                                       Strides os) {
+                                                       Strides os, CutTiles cut) {
   const int sub = threadIdx.x & 31;
   const int64_t step = (int64_t)gridDim.x * 8;
   for (int64_t row = (int64_t)blockIdx.x * 8 + (threadIdx.x >> 5); row < rows; row += step) {
+    int64_t orow = row;             // its index in [B * Hq * Nq]
+    if (cut.tiles) {
+      const int tile = cut.whole + (int)(row >> 8), seq = tile / cut.tiles_q;
+      const int r = (tile - seq * cut.tiles_q) * 256 + (int)(row & 255);
+      if (r >= cut.seq_r) continue;
+      orow = ((int64_t)seq * cut.pack + r % cut.pack) * seq_q + r / cut.pack;
+    }
     float mx = -INFINITY;
     for (int s = sub; s < splits; s += 32) mx = fmaxf(mx, lpart[s * rows + row]);
     mx = max32(mx);
@@ -413,13 +431,13 @@ __global__ void __launch_bounds__(256) fa_merge_kernel(const float* __restrict__
       wsum = sum32(wsum);
     }
     const float inv = wsum > 0.f ? 1.f / wsum : 0.f;
-    const int64_t bh = row / seq_q;
-    const int i = (int)(row - bh * seq_q);
+    const int64_t bh = orow / seq_q;
+    const int i = (int)(orow - bh * seq_q);
     const int b = (int)(bh / heads_q), h = (int)(bh - (int64_t)b * heads_q);
     const h4 out = {(_Float16)(a0 * inv), (_Float16)(a1 * inv), (_Float16)(a2 * inv),
                     (_Float16)(a3 * inv)};
     *reinterpret_cast<h4*>(row_at(o, os, b, h, i) + 4 * sub) = out;
-    if (lse && sub == 0) lse[row] = wsum > 0.f ? mx + __builtin_amdgcn_logf(wsum) * LN2 : -INFINITY;
+    if (lse && sub == 0) lse[orow] = wsum > 0.f ? mx + __builtin_amdgcn_logf(wsum) * LN2 : -INFINITY;
   }
 }
 
@@ -528,6 +546,55 @@ __device__ __forceinline__ void trace_record(const FaArgs& args, int tile, uint6
   rec[7] = (uint64_t)bn;
 }
 
+// Copy of the kernel arguments read from the kernel-argument segment at
+// address `addr` (scalar loads), field by field.
+typedef const FaArgs __attribute__((address_space(4)))* KernargArgs;
+__device__ __forceinline__ Strides load_strides(const Strides __attribute__((address_space(4)))& s) {
+  return Strides{s.b, s.h, s.n};
+}
+__device__ __forceinline__ FaArgs load_args(uint64_t addr) {
+  KernargArgs a = reinterpret_cast<KernargArgs>(addr);
+  FaArgs r;
+  r.q = a->q;
+  r.k = a->k;
+  r.v = a->v;
+  r.o = a->o;
+  r.lse = a->lse;
+  r.stats = a->stats;
+  r.trace = a->trace;
+  r.next_tile = a->next_tile;
+  r.tiles = a->tiles;
+  r.heads_q = a->heads_q;
+  r.group = a->group;
+  r.seq_q = a->seq_q;
+  r.seq_k = a->seq_k;
+  r.nk_valid = a->nk_valid;
+  r.causal = a->causal;
+  r.causal_off = a->causal_off;
+  r.c = a->c;
+  r.qs = load_strides(a->qs);
+  r.ks = load_strides(a->ks);
+  r.os = load_strides(a->os);
+  r.opart = a->opart;
+  r.lpart = a->lpart;
+  r.part_rows = a->part_rows;
+  r.whole = a->whole;
+  r.splits = a->splits;
+  r.direct = a->direct;
+  r.vs = load_strides(a->vs);
+  return r;
+}
+
+// The kernel arguments through an address the compiler cannot follow: read
+// where they are needed, at a tile's start and again for its results, instead
+// of staying live in scalar registers across every key loop, where, at 256
+// VGPRs per wave, that pressure spills.
+__device__ __forceinline__ FaArgs reload_args() {
+  uint64_t addr = reinterpret_cast<uint64_t>(__builtin_amdgcn_kernarg_segment_ptr());
+  asm volatile("" : "+s"(addr));
+  return load_args(addr);
+}
+
 // Ping-pong attention body: 8 waves x 32 query rows (BM = 256), two wave
 // groups of four, one wave of each group per SIMD. The key loop runs in
 // phases separated by workgroup barriers; a wave alternates an MFMA step
@@ -571,7 +638,8 @@ __device__ __forceinline__ void fa_pp_tile(const FaArgs& args, const int tile, c
   constexpr bool CAPTURE = MODE == MODE_CAPTURE;
   constexpr bool TRACE = MODE == MODE_TRACE;
   constexpr bool SYNC = MODE == MODE_SYNC;
-  constexpr bool SPLIT = MODE == MODE_SPLIT;
+  // Whether this item is one of several parts of the tile's keys (uniform).
+  const bool cut = can_cut(MODE) && tile >= args.whole;
   uint64_t real0 = 0, clk0 = 0;
   if constexpr (TRACE) {
     real0 = __builtin_amdgcn_s_memrealtime();
@@ -690,11 +758,11 @@ __device__ __forceinline__ void fa_pp_tile(const FaArgs& args, const int tile, c
     const int kend = pos_of(min(qt * BM + BM, seq_r) - 1) + 1 + args.causal_off;
     nblk = kend <= 0 ? 0 : min(nblk, (kend + BN - 1) / BN);
   }
-  // Split mode: this work item streams key blocks [kb0, kb1) of the tile
-  // (part `split` of args.splits near-equal parts of the key blocks), with
+  // A part streams key blocks [kb0, kb1) of the tile (part `split` of
+  // args.splits near-equal parts of the key blocks), with
   // the loads, limits and masks below relative to key kb0 * BN.
   int kb0 = 0;
-  if constexpr (SPLIT) {
+  if (cut) {
     const int nbt = seq_k / BN;
     kb0 = (int)((int64_t)split * nbt / args.splits);
     const int kb1 = (int)((int64_t)(split + 1) * nbt / args.splits);
@@ -702,7 +770,10 @@ __device__ __forceinline__ void fa_pp_tile(const FaArgs& args, const int tile, c
     klim -= kb0 * BN;
     klim_w -= kb0 * BN;
   }
-  const size_t part = (size_t)split * rows_all + grow;   // split mode: partial row
+  auto part_row = [&](const FaArgs& args) {     // this lane's row of opart and lpart
+    return (size_t)split * args.part_rows +
+           (args.whole == 0 ? grow : (size_t)(tile - args.whole) * BM + wave_u * 32 + l32);
+  };
   if (nblk == 0) {
     // No row of this tile sees a key (bottom-right mask, Nq > Nk): O = 0 and
     // lse = -inf. Uniform over the workgroup, before any barrier or load.
@@ -718,10 +789,12 @@ __device__ __forceinline__ void fa_pp_tile(const FaArgs& args, const int tile, c
         }
       }
     }
-    if constexpr (TRACE) trace_record(args, tile, real0, clk0, 0, BN);
+    if constexpr (TRACE)
+      if (split == 0) trace_record(args, tile, real0, clk0, 0, BN);
     if (!row_ok) return;
-    if constexpr (SPLIT) {
+    if (cut) {
       // The part's lse is -inf and its O row zeros (weight 0 in the merge).
+      const size_t part = part_row(args);
       if (hf == 0) args.lpart[part] = -INFINITY;
       float* prow = args.opart + part * HD;
       const float4 zero = {0.f, 0.f, 0.f, 0.f};
@@ -1243,7 +1316,8 @@ __device__ __forceinline__ void fa_pp_tile(const FaArgs& args, const int tile, c
   // Every wave has waited for its loads before the last barrier, so nothing
   // writes the ring any more, and nobody reads it.
   claim();
-  if constexpr (TRACE) trace_record(args, tile, real0, clk0, nblk, BN);
+  if constexpr (TRACE)
+    if (split == 0) trace_record(args, tile, real0, clk0, nblk, BN);
 
   if constexpr (CAPTURE) {
     // Key blocks past the causal diagonal leave every statistic unchanged.
@@ -1267,12 +1341,14 @@ __device__ __forceinline__ void fa_pp_tile(const FaArgs& args, const int tile, c
   // that saw no key (causal mask) has l = 0: O = 0 and lse = -inf.
   const float l = half_sum(lsum);
   const float inv = l > 0.f ? 1.f / l : 0.f;
-  if constexpr (SPLIT) {
+  const FaArgs fin = reload_args();
+  if (cut) {
     if (!row_ok) return;
+    const size_t part = part_row(fin);
     // This part's O / l in FP32 and its log-sum-exp (-inf, with O = 0, for a
     // row that sees no key of the part).
-    if (hf == 0) args.lpart[part] = (__builtin_amdgcn_logf(l) + m * c) * LN2;
-    float* prow = args.opart + part * HD;
+    if (hf == 0) fin.lpart[part] = (__builtin_amdgcn_logf(l) + m * c) * LN2;
+    float* prow = fin.opart + part * HD;
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
@@ -1283,7 +1359,7 @@ __device__ __forceinline__ void fa_pp_tile(const FaArgs& args, const int tile, c
       }
     return;
   }
-  if (args.lse && hf == 0 && row_ok) args.lse[grow] = (__builtin_amdgcn_logf(l) + m * c) * LN2;
+  if (fin.lse && hf == 0 && row_ok) fin.lse[grow] = (__builtin_amdgcn_logf(l) + m * c) * LN2;
   // A lane holds 4 dims here and there of one row; stored like that, a store
   // instruction touches 32 rows in 16-byte pieces, which left 5.3 us between a
   // workgroup's tiles (2.8 now; B=4, 32 heads, 2048 causal keys: 172.1 -> 164.7
@@ -1304,14 +1380,14 @@ __device__ __forceinline__ void fa_pp_tile(const FaArgs& args, const int tile, c
       *reinterpret_cast<h4*>(rows + l32 * 256 + (((4 * dt + g) ^ (l32 & 15)) << 4) + hf * 8) = out;
     }
   }
-  const int64_t obase = (int64_t)b * args.os.b + (int64_t)head_of(rowc) * args.os.h +
-                        (int64_t)pos_of(rowc) * args.os.n;   // this lane's row in o
+  const int64_t obase = (int64_t)b * fin.os.b + (int64_t)head_of(rowc) * fin.os.h +
+                        (int64_t)pos_of(rowc) * fin.os.n;   // this lane's row in o
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     const int r = 4 * i + (lane >> 4);
     const u32x4 val = *reinterpret_cast<const u32x4*>(rows + r * 256 + (((lane & 15) ^ (r & 15)) << 4));
     const int64_t at = (int64_t)(uint32_t)__shfl((int)obase, r) | (int64_t)__shfl((int)(obase >> 32), r) << 32;
-    if (qt * BM + wave_u * 32 + r < seq_r) *reinterpret_cast<u32x4*>(o + at + (lane & 15) * 8) = val;
+    if (qt * BM + wave_u * 32 + r < seq_r) *reinterpret_cast<u32x4*>(fin.o + at + (lane & 15) * 8) = val;
   }
 }
 
@@ -1334,64 +1410,24 @@ __device__ __forceinline__ void fa_pp_tile(const FaArgs& args, const int tile, c
 // never larger than the item count), and then workgroup i takes item i / 8 of
 // queue i % 8 (consecutive workgroups go to different dies) without the
 // counters, so such a launch needs no counter reset.
-// Copy of the kernel arguments read from the kernel-argument segment at
-// address `addr` (scalar loads), field by field.
-typedef const FaArgs __attribute__((address_space(4)))* KernargArgs;
-__device__ __forceinline__ Strides load_strides(const Strides __attribute__((address_space(4)))& s) {
-  return Strides{s.b, s.h, s.n};
-}
-__device__ __forceinline__ FaArgs load_args(uint64_t addr) {
-  KernargArgs a = reinterpret_cast<KernargArgs>(addr);
-  FaArgs r;
-  r.q = a->q;
-  r.k = a->k;
-  r.v = a->v;
-  r.o = a->o;
-  r.lse = a->lse;
-  r.stats = a->stats;
-  r.trace = a->trace;
-  r.next_tile = a->next_tile;
-  r.tiles = a->tiles;
-  r.heads_q = a->heads_q;
-  r.group = a->group;
-  r.seq_q = a->seq_q;
-  r.seq_k = a->seq_k;
-  r.nk_valid = a->nk_valid;
-  r.causal = a->causal;
-  r.causal_off = a->causal_off;
-  r.c = a->c;
-  r.qs = load_strides(a->qs);
-  r.ks = load_strides(a->ks);
-  r.os = load_strides(a->os);
-  r.opart = a->opart;
-  r.lpart = a->lpart;
-  r.splits = a->splits;
-  r.vs = load_strides(a->vs);
-  return r;
-}
-
 template <bool ACC16, int BN, int NS, int MODE, bool PACKED, bool VNAT>
 __device__ __forceinline__ void fa_pp_body(const FaArgs& args) {
   __shared__ int claimed[2][2];                  // queue and item of this and the next round
-  // Work items: query tiles, or in split mode (part, tile) pairs, the tiles
-  // of one part consecutive (they read the same keys).
-  const int tiles = args.tiles;
-  int items = tiles;
-  if constexpr (MODE == MODE_SPLIT) items *= args.splits;
-  // Queue x holds items / 8 items, and one more for x < items % 8.
-  auto count = [&](int x) { return (items >> 3) + (x < (items & 7) ? 1 : 0); };
-  const bool direct = items <= (int)gridDim.x;   // one workgroup per item
-  // The thread index and the arguments' address pass through opaque moves, so
-  // nothing derived from them stays in registers across a tile's key loop.
+  // Work items: whole tiles, then (part, tile) pairs of the cut tiles, the
+  // tiles of one part consecutive (they read the same keys). Queue x holds an
+  // eighth of each kind, consecutive ones, and one more of the first n % 8.
+  const int tiles = args.tiles, whole = can_cut(MODE) ? args.whole : tiles;
+  const int cuts = can_cut(MODE) ? (tiles - whole) * args.splits : 0;
+  auto share = [](int n, int x) { return (n >> 3) + (x < (n & 7) ? 1 : 0); };
+  auto start = [](int n, int x) { return x * (n >> 3) + min(x, n & 7); };
+  auto count = [&](int x) { return share(whole, x) + share(cuts, x); };
+  const bool direct = args.direct;
+  // The thread index passes through an opaque move, so nothing derived from it
+  // stays in registers across a tile's key loop.
   auto thread = []() {
     int tid;
     asm volatile("v_mov_b32 %0, %1" : "=v"(tid) : "v"((int)threadIdx.x));
     return tid;
-  };
-  auto kernargs = []() {
-    uint64_t addr = reinterpret_cast<uint64_t>(__builtin_amdgcn_kernarg_segment_ptr());
-    asm volatile("" : "+s"(addr));
-    return addr;
   };
   // XCC_ID (id 20): the die.
   auto die = []() { return (int)(__builtin_amdgcn_s_getreg((31 << 11) | 20) & (kQueues - 1)); };
@@ -1439,19 +1475,16 @@ __device__ __forceinline__ void fa_pp_body(const FaArgs& args) {
       i = __builtin_amdgcn_readfirstlane(claimed[n & 1][1]);
       if (x < 0) break;
     }
-    // Each tile reloads the arguments from the kernel-argument segment: kept
-    // from one tile to the next, all of them would stay live in scalar
-    // registers across every key loop, and at 256 VGPRs per wave that
-    // pressure spills.
-    const FaArgs a = load_args(kernargs());
-    // Without a mask (and in split mode) the queues are consecutive runs of
-    // the item order, in which the tiles of one KV head follow each other. A
-    // causal mask's tiles go out longest first: queue x then holds an eighth
-    // of the sequences, or, if 8 does not divide them, every eighth tile.
-    int tile = x * (items >> 3) + min(x, items & 7) + i, split = 0;
-    if constexpr (MODE == MODE_SPLIT) {
-      split = tile / tiles;
-      tile -= split * tiles;
+    const FaArgs a = reload_args();
+    // A causal mask's whole tiles go out longest first: queue x then holds an
+    // eighth of the sequences, or, if 8 does not divide them, every eighth
+    // tile.
+    const int nw = share(whole, x);
+    int tile = start(whole, x) + i, split = 0;
+    if (can_cut(MODE) && i >= nw) {
+      const int at = start(cuts, x) + i - nw;
+      split = at / (tiles - whole);
+      tile = whole + at - split * (tiles - whole);
     } else if (a.causal) {
       const int rows = PACKED ? a.seq_q * a.group : a.seq_q;
       const int nbh = tiles / ((rows + 255) / 256), nb = nbh >> 3;
@@ -1815,7 +1848,7 @@ constexpr uint64_t kCounterBytes = 256;
 #define FA_MODES(KERNEL, BN, NS, PK, VN)                                                    \
   {&KERNEL<BN, NS, MODE_RUN, PK, VN>, &KERNEL<BN, NS, MODE_CAPTURE, PK, VN>,                 \
    &KERNEL<BN, NS, MODE_TRACE, PK, VN>, &KERNEL<BN, NS, MODE_SYNC, PK, VN>,                  \
-   &KERNEL<BN, NS, MODE_SPLIT, PK, VN>}
+   &KERNEL<BN, NS, MODE_PARTS, PK, VN>}
 #define FA_TILE(NAME, BN, NS, VN)                                                           \
   TileConfig {                                                                              \
     NAME, BN, VN, pp_lds_bytes(BN, NS, VN), {                                               \
@@ -1975,6 +2008,52 @@ const attn_fn kRowsFn[2][2] = {   // [packed][acc]
     {&hip_fa_fp32acc_rows_kernel<false>, &hip_fa_fp16acc_rows_kernel<false>},
     {&hip_fa_fp32acc_rows_kernel<true>, &hip_fa_fp16acc_rows_kernel<true>},
 };
+
+// A one-pass launch runs its tiles in rounds of one per CU, and a last round
+// of few tiles takes as long as a full one: 564 tiles of 61 key blocks on 256
+// CUs kept 204 of them idle for a quarter of the launch. The tiles of the
+// last, partial round are therefore cut into parts of their key range, which
+// spread over all CUs, and the merge kernel combines them (full attention on
+// the automatic tile only; a causal launch's last tiles are short). The
+// number of parts is the one with the shortest modelled launch: a key block
+// takes 2 us on a CU with the others idle and 3.4 us with all of them busy
+// (the power limit), an item 2.5 blocks on top of its own, the merge its
+// bytes at 4 TB/s and 5 us; it must win 3 %. The choice takes 256 CUs for
+// granted, as the workspace is sized without a device, and cuts only what
+// fa_fwd_noalloc's scratch holds together with the rest of the workspace, so
+// that both run the same kernels. A launch of less than one round is not cut:
+// its parts would cost more than they save at 192 tiles, and few tiles
+// against long keys have the key-split forward.
+constexpr int kPlanCus = 256;
+struct CutPlan {
+  int64_t whole, cut;      // tiles
+  int parts;
+  uint64_t rows() const { return (uint64_t)cut * kRows; }
+  uint64_t lpart_bytes() const { return parts > 1 ? parts * rows() * sizeof(float) : 0; }
+  uint64_t bytes() const { return lpart_bytes() * (1 + HD); }
+};
+// Measured: B=2, 24 heads on 2 KV heads, 3001 x 7777, FP16 O (564 tiles, 52
+// cut into 4 parts): 593 -> 532 us.
+CutPlan cut_plan(const fa_problem* p, const TileConfig* tile, const KeyLayout& lay) {
+  const int64_t tiles = (int64_t)grid_size(p), rem = tiles % kPlanCus;
+  CutPlan plan{tiles, 0, 1};
+  if (p->kernel != 0 || p->causal != FA_CAUSAL_NONE || tiles < kPlanCus || rem == 0) return plan;
+  const double nbt = (double)(lay.nk_pad / tile->keys) * (tile->keys / 128.0), item = 2.5;
+  auto block_us = [](double active) { return 2.0 + 1.4 * std::min(1.0, active / kPlanCus); };
+  const double whole_us = (double)(tiles / kPlanCus) * (nbt + item) * block_us(kPlanCus);
+  double best = 0.97 * (whole_us + (nbt + item) * block_us((double)rem));
+  for (int s = 2; s <= 16 && s <= nbt; ++s) {
+    const double items = (double)rem * s, rows = (double)rem * kRows;
+    const double t = whole_us + ceil(items / kPlanCus) * (ceil(nbt / s) + item) * block_us(items) + 5.0 +
+                     rows * (s * (HD + 1) * 4.0 + (HD * 2 + 4)) / 4e6;
+    const CutPlan c{tiles - rem, rem, s};
+    if (t < best && lay.workspace_bytes() + c.bytes() <= FA_NOALLOC_SCRATCH_BYTES) {
+      best = t;
+      plan = c;
+    }
+  }
+  return plan;
+}
 
 // Split mode's partial results, after the work queues in the workspace:
 // the parts' log-sum-exp (FP32 [splits][R], R = B * Hq * Nq) from a 256-byte
@@ -2268,21 +2347,25 @@ int launch(const fa_problem* p, const fa_strides* strides, const void* q, const 
   const SplitLayout sl = split_layout(p, lay, splits);
   if (!workspace || workspace_bytes < (splits > 1 ? sl.end : lay.workspace_bytes()))
     return FA_ERR_WORKSPACE;
+  // The last round's tiles, cut, where the workspace has room for their parts.
+  const int64_t tiles = (int64_t)grid_size(p);
+  CutPlan plan{tiles, 0, 1};
+  if (splits <= 1 && !ex.stats) {
+    plan = cut_plan(p, tile, lay);
+    if (workspace_bytes < lay.workspace_bytes() + plan.bytes()) plan = CutPlan{tiles, 0, 1};
+  }
   for (const void* ptr : {q, k, v, (const void*)o, (const void*)workspace, (const void*)ex.lse,
                           (const void*)ex.stats, (const void*)ex.trace})
     if (reinterpret_cast<uintptr_t>(ptr) & 15) return FA_ERR_ALIGN;
   if (ex.stats && ex.stats_count < capture_count(p, tile, lay)) return FA_ERR_CAPTURE;
   if (ex.trace && ex.trace_count < grid_size(p) * TRACE_WORDS) return FA_ERR_TRACE;
   const int acc = p->acc == FA_ACC_FP16 ? 1 : 0;
-  const int mode = splits > 1 ? MODE_SPLIT
-                   : ex.stats ? MODE_CAPTURE
-                   : ex.trace ? MODE_TRACE
-                   : ex.sync  ? MODE_SYNC
-                              : MODE_RUN;
+  const int mode = ex.stats ? MODE_CAPTURE : ex.trace ? MODE_TRACE : ex.sync ? MODE_SYNC
+                   : splits > 1 || plan.parts > 1 ? MODE_PARTS : MODE_RUN;
   const int packed = row_layout(p).pack > 1 ? 1 : 0;
   rc = check_stream_device(stream);
   if (rc) return rc;
-  const bool rows_kernel = mode == MODE_SPLIT && few_rows(p, splits);
+  const bool rows_kernel = splits > 1 && few_rows(p, splits);
   const attn_fn fn = rows_kernel ? kRowsFn[packed][acc] : tile->fn[packed][acc][mode];
   const int lds = rows_kernel ? kRowsLds : tile->lds;
   rc = ensure_lds_limit(fn, lds, rows_kernel ? kNumTiles : (int)(tile - kTiles), packed, acc, mode);
@@ -2302,14 +2385,18 @@ int launch(const fa_problem* p, const fa_strides* strides, const void* q, const 
   _Float16* kpad = copies ? ws + (lay.vnat ? 0 : head_elems) : nullptr;
   _Float16* vpad = copies && lay.vnat ? kpad + head_elems : nullptr;
   int* next_tile = reinterpret_cast<int*>(static_cast<char*>(workspace) + lay.counter_offset());
+  // Work items, and whether each gets a workgroup of its own.
+  const uint64_t items = splits > 1 ? (uint64_t)tiles * splits : (uint64_t)(plan.whole + plan.cut * plan.parts);
+  const bool direct = rows_kernel || (items <= (uint64_t)cus && plan.cut == 0);
 
   // hipLaunchKernel returns the status of this launch alone; errors left
   // pending by the caller's earlier work are neither read nor cleared.
   if (mode == MODE_SYNC) {
-    // Sync mode: the workspace (V^T, padded K and V) starts as FP16 NaN, so a read
-    // of any element the prep kernel does not write reaches the output.
+    // Sync mode: the workspace starts as FP16 NaN, so a read of any element of
+    // V^T, the padded K and V or a cut tile's parts that nothing has written
+    // reaches the output (the prep kernel resets the work queues after this).
     u32x4* ws = static_cast<u32x4*>(workspace);
-    uint64_t n16 = lay.counter_offset() / 16;
+    uint64_t n16 = (lay.workspace_bytes() + plan.bytes()) / 16;
     void* poison_args[] = {&ws, &n16};
     const unsigned blocks = (unsigned)std::min<uint64_t>((n16 + 255) / 256, 4096);
     if (n16 && hipLaunchKernel(reinterpret_cast<const void*>(&fa_poison_kernel), dim3(blocks),
@@ -2326,7 +2413,6 @@ int launch(const fa_problem* p, const fa_strides* strides, const void* q, const 
     // The natural-V tile without copies needs the pad kernel only for
     // the counter, which a launch of at most one work item per CU does not
     // use (fa_pp_body): then nothing runs before the attention kernel.
-    const bool direct = rows_kernel || grid_size(p) * splits <= (uint64_t)cus;
     bool ok = true;
     if (!lay.vnat)
       ok = hipLaunchKernel(reinterpret_cast<const void*>(&fa_prep_kernel), groups, dim3(256),
@@ -2345,11 +2431,17 @@ int launch(const fa_problem* p, const fa_strides* strides, const void* q, const 
   args.lse = ex.lse;
   args.stats = ex.stats;
   args.trace = ex.trace;
-  args.opart = reinterpret_cast<float*>(static_cast<char*>(workspace) + sl.opart_offset);
+  const bool cut = plan.parts > 1;
   args.lpart = reinterpret_cast<float*>(static_cast<char*>(workspace) + sl.lpart_offset);
+  args.opart = reinterpret_cast<float*>(
+      static_cast<char*>(workspace) +
+      (cut ? sl.lpart_offset + plan.lpart_bytes() : sl.opart_offset));
+  args.part_rows = cut ? (int64_t)plan.rows() : p->batch * p->heads_q * p->seq_q;
+  args.whole = splits > 1 ? 0 : (int)plan.whole;
+  args.direct = direct;
   args.next_tile = next_tile;
   args.tiles = (int)(rows_kernel ? row_tiles(p) : grid_size(p));
-  args.splits = splits;
+  args.splits = cut ? plan.parts : splits;
   args.heads_q = (int)p->heads_q;
   args.group = (int)(p->heads_q / p->heads_kv);
   args.seq_q = (int)p->seq_q;
@@ -2370,20 +2462,23 @@ int launch(const fa_problem* p, const fa_strides* strides, const void* q, const 
   const uint64_t kv_heads = (uint64_t)(p->batch * p->heads_kv);
   const unsigned grid =
       rows_kernel ? (unsigned)((kv_heads * splits + 7) / 8 * 8 * (args.tiles / kv_heads))
-                  : (unsigned)std::min<uint64_t>(grid_size(p) * splits, (uint64_t)cus);
+                  : (unsigned)std::min<uint64_t>(items, (uint64_t)cus);
   if (hipLaunchKernel(reinterpret_cast<const void*>(fn), dim3(grid), dim3(kThreads), attn_args, lds,
                       st) != hipSuccess)
     return FA_ERR_LAUNCH;
-  if (splits > 1) {
+  if (args.splits > 1) {
     const float* opart = args.opart;
     const float* lpart = args.lpart;
     _Float16* out = args.o;
     float* lse = ex.lse;
-    int nsplit = splits;
-    int64_t rows = p->batch * p->heads_q * p->seq_q;
+    int nsplit = args.splits;
+    int64_t rows = args.part_rows;
     int heads_q = (int)p->heads_q, seq_q = (int)p->seq_q;
-    void* merge_args[] = {&opart, &lpart, &out, &lse, &nsplit, &rows, &heads_q, &seq_q, &os};
-    const bool wide = merge_wide(rows, splits);
+    const RowLayout rl = row_layout(p);
+    CutTiles cuts{(int)plan.cut, (int)plan.whole, (int)((rl.rows + kRows - 1) / kRows), (int)rl.pack,
+                  (int)rl.rows};
+    void* merge_args[] = {&opart, &lpart, &out, &lse, &nsplit, &rows, &heads_q, &seq_q, &os, &cuts};
+    const bool wide = !cut && merge_wide(rows, splits);
     const unsigned blocks =
         (unsigned)std::min<int64_t>(wide ? rows : (rows + 7) / 8, (int64_t)1 << 20);
     const void* merge_fn = wide ? reinterpret_cast<const void*>(&fa_merge_wide_kernel)
@@ -2445,7 +2540,7 @@ int fa_fwd_workspace_bytes(const fa_problem* p, uint64_t* bytes) {
   int rc = validate(p, &tile);
   if (rc) return rc;
   const KeyLayout lay = key_layout(p, tile);
-  *bytes = lay.workspace_bytes();
+  *bytes = lay.workspace_bytes() + cut_plan(p, tile, lay).bytes();
   return FA_OK;
 }
 
@@ -2569,7 +2664,7 @@ int fa_fwd_split_workspace_bytes(const fa_problem* p, int32_t splits, uint64_t* 
   int s = 0;
   rc = resolve_splits(p, tile, lay, splits, cus, &s);
   if (rc) return rc;
-  *bytes = s > 1 ? split_layout(p, lay, s).end : lay.workspace_bytes();
+  *bytes = s > 1 ? split_layout(p, lay, s).end : lay.workspace_bytes() + cut_plan(p, tile, lay).bytes();
   return FA_OK;
 }
 

@@ -119,15 +119,16 @@ typedef struct fa_problem {
 
 /*
  * Bytes of device workspace fa_fwd() needs for problem *p: 256 bytes for the
- * counter the kernel's workgroups take query tiles from, plus, for a tile
+ * queues the kernel's workgroups take query tiles from, plus, for a tile
  * that reads V^T (see V layouts above), V^T (B * Hkv * Nk' * 256 bytes), and,
  * with a ragged key tail, room for zero-padded copies to a whole key block of
  * the selected tile (Nk' keys) of k (V^T tiles) or of k and v
  * (pp_n128_r2_vnat), B * Hkv * Nk' * 256 bytes each (written only when the
  * rows of k or v lie so far apart that Nk' of them span 2 GiB or more;
- * otherwise a ragged tail is read in place). pp_n128_r2_vnat without a key tail reads k
- * and v where they lie and needs the 256-byte counter alone. Replaces phase 1 of the
- * reference's operator call,
+ * otherwise a ragged tail is read in place), and, for a launch whose last
+ * round of tiles is cut (see fa_fwd()), the parts' results. pp_n128_r2_vnat
+ * without a key tail reads k and v where they lie and needs the 256-byte
+ * queue slot alone. Replaces phase 1 of the reference's operator call,
  * aclnn<Op>GetWorkspaceSize (backends/cce_fa_nk_nz_vector_fp32_v5_sumpack/
  * binding.py:21-24,74-75), whose host tiling sizes the scratch buffer
  * (project/op_host/fa_fa_nk_nz_vector_fp32_v5_sumpack.cpp:52-87).
@@ -141,6 +142,14 @@ int fa_fwd_workspace_bytes(const fa_problem* p, uint64_t* bytes);
  * binding.py:25-27,80), and the external reference op it is checked against
  * (backends/npu_fa/backend.py:36-49). The workspace must hold at least
  * fa_fwd_workspace_bytes(p) bytes; its contents on entry do not matter.
+ *
+ * Full attention on the automatic tile with more than 256 query tiles, not a
+ * multiple of 256, may cut the tiles of its last, partial round (tile count
+ * modulo 256, the last ones) into parts of their key range, so that they
+ * occupy every CU, and combine the parts as fa_fwd_split() does: those rows
+ * then differ from an uncut launch's by FP32 summation order. This is a
+ * function of the problem alone; with a workspace that holds all else but
+ * not the parts, nothing is cut.
  */
 int fa_fwd(const fa_problem* p, const void* q, const void* k, const void* v, void* o,
            void* workspace, uint64_t workspace_bytes, void* stream);
@@ -218,7 +227,8 @@ int fa_fwd_capture(const fa_problem* p, const void* q, const void* k, const void
  *   3  s_memtime when the tile starts (shader clock cycles)
  *   4  s_memtime after its key loop
  *   5  tile index w
- *   6  key blocks streamed
+ *   6  key blocks streamed (of a cut tile, and all of its record: its first
+ *      part's)
  *   7  keys per block
  * so the shader clock the tile ran at is (w4 - w3) / (w2 - w1) * 100
  * MHz. The trace kernel is a separate instantiation of the same tile (the
