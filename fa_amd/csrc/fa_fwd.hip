@@ -1810,7 +1810,7 @@ constexpr int pp_lds_bytes(int bn, int ns, bool vnat) {
 // Device entry points, one per accumulation variant. Their names contain the
 // backend names of the two accumulation variants, which is how a profile
 // attributes kernel time to a backend. Template parameters: BN keys per
-// block, NS slots in the LDS ring, MODE (production, capture, trace, sync or split;
+// block, NS slots in the LDS ring, MODE (production, capture, trace, sync or parts;
 // each mode is a separate kernel, so the production kernels carry none of
 // the debug code), PACKED (tiles of packed rows: the group's query heads
 // position by position, see fa_pp_tile; also separate kernels, so the
@@ -1878,7 +1878,8 @@ constexpr int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]);
 // few query rows per KV head (G * Nq, G = Hq / Hkv). Timed against each
 // other (automatic split count, one session), natural V was 5 % faster at
 // 1536 rows per KV head and 4-12 % slower from 3072 up; the switch sits at
-// kNaturalVRows.
+// kNaturalVRows. One-pass launches of short sequences run natural V above it
+// too (natural_is_shorter).
 constexpr int kAutoVt = 3;
 constexpr int kAutoNatural = 4;
 constexpr int64_t kNaturalVRows = 2048;
@@ -2230,6 +2231,29 @@ bool rows_in_place(int64_t n, int64_t nk_pad) {
   return n < lim && n * nk_pad < lim;
 }
 
+// Whether a one-pass launch of the automatic V^T tile runs its natural-V twin
+// (the same values bit for bit, see the table above): where every tile has a
+// workgroup of its own and V is read in place, nothing then runs before the
+// attention kernel. That saves the prep launch, 3 us and V's bytes twice at
+// 4.7 TB/s, and costs the second operand read of every key block, 0.27 us a
+// block while few CUs are busy and less as they fill up (the power limit
+// sets the pace there). Fitted to both tiles over 12 to 256 tiles (V^T /
+// natural): 12 heads on one KV head, 256 keys 14.0 / 11.7 us, 512 18.5 /
+// 16.5, 1000 27.7 / 26.6, 2048 45.5 / 46.0; 16 KV heads, 3000 keys 83.3 /
+// 75.7, 4096 130.9 / 123.9; 64 heads on 8 KV heads, 1024 rows by 8192 keys
+// 242.3 / 239.5. At 256 blocks natural V was the slower one for every head
+// count (by 1.6 to 13 %), so the fit stops at kShortBlocks.
+constexpr int64_t kShortBlocks = 64;
+bool natural_is_shorter(const fa_problem* p, const KeyLayout& lay, const Strides& ks,
+                        const Strides& vs, int64_t tiles, int cus) {
+  const int64_t blocks = lay.nk_pad / 128;
+  if (tiles > cus || blocks > kShortBlocks || !rows_in_place(ks.n, lay.nk_pad) ||
+      !rows_in_place(vs.n, lay.nk_pad))
+    return false;
+  const double saved = 3.0 + (double)(p->batch * p->heads_kv * lay.nk_pad) * (2 * HD * sizeof(_Float16)) / 4.7e6;
+  return saved > 1.15 * (double)blocks * (0.27 - 0.15 * (double)tiles / cus);
+}
+
 // Caller strides must keep every 128-element row 16-byte aligned and rows
 // apart (n >= 128); the K rows of one head, and its V rows if the tile reads
 // them in place (natural-V tile), must span less than 2^31 bytes (32-bit
@@ -2321,7 +2345,7 @@ int launch(const fa_problem* p, const fa_strides* strides, const void* q, const 
   int rc = validate(p, &tile);
   if (rc) return rc;
   if (!q || !k || !v || !o) return FA_ERR_NULL;
-  const KeyLayout lay = key_layout(p, tile);
+  KeyLayout lay = key_layout(p, tile);
   Strides qs = contiguous(p->heads_q, p->seq_q), os = qs;
   Strides ks = contiguous(p->heads_kv, p->seq_k), vs = ks;
   if (strides) {
@@ -2365,15 +2389,27 @@ int launch(const fa_problem* p, const fa_strides* strides, const void* q, const 
   const int packed = row_layout(p).pack > 1 ? 1 : 0;
   rc = check_stream_device(stream);
   if (rc) return rc;
+  if (!cus) {
+    rc = device_cus(&cus);
+    if (rc) return rc;
+  }
+  if (p->kernel == 0 && splits <= 1 && !lay.vnat) {
+    // Both twins are set up by the first call of either: a later call may
+    // have to make do without set-up (graph capture).
+    const TileConfig* twin = &kTiles[kAutoNatural - 1];
+    rc = ensure_lds_limit(twin->fn[packed][acc][mode], twin->lds, kAutoNatural - 1, packed, acc, mode);
+    if (!rc) rc = ensure_lds_limit(tile->fn[packed][acc][mode], tile->lds, (int)(tile - kTiles), packed, acc, mode);
+    if (rc) return rc;
+    if (natural_is_shorter(p, lay, ks, vs, tiles, cus)) {
+      tile = twin;
+      lay = key_layout(p, tile);       // needs no more workspace than the V^T tile's
+    }
+  }
   const bool rows_kernel = splits > 1 && few_rows(p, splits);
   const attn_fn fn = rows_kernel ? kRowsFn[packed][acc] : tile->fn[packed][acc][mode];
   const int lds = rows_kernel ? kRowsLds : tile->lds;
   rc = ensure_lds_limit(fn, lds, rows_kernel ? kNumTiles : (int)(tile - kTiles), packed, acc, mode);
   if (rc) return rc;
-  if (!cus) {
-    rc = device_cus(&cus);
-    if (rc) return rc;
-  }
 
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   // Workspace: [V^T] [padded K] [padded V] counter, as the layout has them.

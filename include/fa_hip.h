@@ -273,7 +273,10 @@ int fa_fwd_tile(const fa_problem* p, int32_t* rows, int32_t* keys);
  * Tile configuration (1..fa_kernel_count()) fa_fwd() would launch for *p,
  * with p->kernel == 0 resolved to the automatic choice. Lets a caller name
  * the kernel it timed, as the reference's profiler identifies a backend's
- * device kernel by name (core/profiler.py:14-25).
+ * device kernel by name (core/profiler.py:14-25). With the automatic choice
+ * a launch may run a variant whose kernels carry the same name: the natural-V
+ * twin of pp_n128_r2 where the sequences are short (equal bit for bit), or the
+ * few-row kernel in fa_fwd_split().
  */
 int fa_fwd_select(const fa_problem* p, int32_t* kernel);
 
