@@ -1878,7 +1878,7 @@ constexpr int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]);
 // few query rows per KV head (G * Nq, G = Hq / Hkv). Timed against each
 // other (automatic split count, one session), natural V was 5 % faster at
 // 1536 rows per KV head and 4-12 % slower from 3072 up; the switch sits at
-// kNaturalVRows. One-pass launches of short sequences run natural V above it
+// kNaturalVRows. Launches of short sequences or parts run natural V above it
 // too (natural_is_shorter).
 constexpr int kAutoVt = 3;
 constexpr int kAutoNatural = 4;
@@ -2231,9 +2231,9 @@ bool rows_in_place(int64_t n, int64_t nk_pad) {
   return n < lim && n * nk_pad < lim;
 }
 
-// Whether a one-pass launch of the automatic V^T tile runs its natural-V twin
-// (the same values bit for bit, see the table above): where every tile has a
-// workgroup of its own and V is read in place, nothing then runs before the
+// Whether a launch of the automatic V^T tile runs its natural-V twin (the
+// same values bit for bit, see the table above): where every work item (a
+// tile, or a part of its key blocks) has a workgroup of its own and V is read in place, nothing then runs before the
 // attention kernel. That saves the prep launch, 3 us and V's bytes twice at
 // 4.7 TB/s, and costs the second operand read of every key block, 0.27 us a
 // block while few CUs are busy and less as they fill up (the power limit
@@ -2242,16 +2242,19 @@ bool rows_in_place(int64_t n, int64_t nk_pad) {
 // 16.5, 1000 27.7 / 26.6, 2048 45.5 / 46.0; 16 KV heads, 3000 keys 83.3 /
 // 75.7, 4096 130.9 / 123.9; 64 heads on 8 KV heads, 1024 rows by 8192 keys
 // 242.3 / 239.5. At 256 blocks natural V was the slower one for every head
-// count (by 1.6 to 13 %), so the fit stops at kShortBlocks.
+// count (by 1.6 to 13 %), so the fit stops at kShortBlocks. Split launches:
+// 256 rows of 12 heads behind 32768 keys in 21 parts 69.0 / 66.5, behind
+// 131072 209.6 / 206.8, 512 rows of 32 heads on 8 behind 8192 in 4 parts 86.0 /
+// 81.8.
 constexpr int64_t kShortBlocks = 64;
 bool natural_is_shorter(const fa_problem* p, const KeyLayout& lay, const Strides& ks,
-                        const Strides& vs, int64_t tiles, int cus) {
-  const int64_t blocks = lay.nk_pad / 128;
-  if (tiles > cus || blocks > kShortBlocks || !rows_in_place(ks.n, lay.nk_pad) ||
+                        const Strides& vs, int64_t items, int splits, int cus) {
+  const int64_t blocks = (lay.nk_pad / 128 + splits - 1) / splits;
+  if (items > cus || blocks > kShortBlocks || !rows_in_place(ks.n, lay.nk_pad) ||
       !rows_in_place(vs.n, lay.nk_pad))
     return false;
   const double saved = 3.0 + (double)(p->batch * p->heads_kv * lay.nk_pad) * (2 * HD * sizeof(_Float16)) / 4.7e6;
-  return saved > 1.15 * (double)blocks * (0.27 - 0.15 * (double)tiles / cus);
+  return saved > 1.15 * (double)blocks * (0.27 - 0.15 * (double)items / cus);
 }
 
 // Caller strides must keep every 128-element row 16-byte aligned and rows
@@ -2368,7 +2371,7 @@ int launch(const fa_problem* p, const fa_strides* strides, const void* q, const 
     rc = resolve_splits(p, tile, lay, ex.splits, cus ? cus : 1, &splits);
     if (rc) return rc;
   }
-  const SplitLayout sl = split_layout(p, lay, splits);
+  SplitLayout sl = split_layout(p, lay, splits);
   if (!workspace || workspace_bytes < (splits > 1 ? sl.end : lay.workspace_bytes()))
     return FA_ERR_WORKSPACE;
   // The last round's tiles, cut, where the workspace has room for their parts.
@@ -2393,16 +2396,17 @@ int launch(const fa_problem* p, const fa_strides* strides, const void* q, const 
     rc = device_cus(&cus);
     if (rc) return rc;
   }
-  if (p->kernel == 0 && splits <= 1 && !lay.vnat) {
+  if (p->kernel == 0 && !lay.vnat) {
     // Both twins are set up by the first call of either: a later call may
     // have to make do without set-up (graph capture).
     const TileConfig* twin = &kTiles[kAutoNatural - 1];
     rc = ensure_lds_limit(twin->fn[packed][acc][mode], twin->lds, kAutoNatural - 1, packed, acc, mode);
     if (!rc) rc = ensure_lds_limit(tile->fn[packed][acc][mode], tile->lds, (int)(tile - kTiles), packed, acc, mode);
     if (rc) return rc;
-    if (natural_is_shorter(p, lay, ks, vs, tiles, cus)) {
+    if (natural_is_shorter(p, lay, ks, vs, tiles * splits, splits, cus)) {
       tile = twin;
       lay = key_layout(p, tile);       // needs no more workspace than the V^T tile's
+      sl = split_layout(p, lay, splits);
     }
   }
   const bool rows_kernel = splits > 1 && few_rows(p, splits);

@@ -1,6 +1,6 @@
-"""Short one-pass launches of the automatic tile equal the V^T tile.
+"""Short launches of the automatic tile equal the V^T tile.
 
-Where every tile has a workgroup of its own and the keys are few, the
+Where every tile, or part of one, has a workgroup of its own and the keys are few, the
 automatic choice reads V in its natural layout instead of running the prep
 kernel first. Both give the same values in the same order, so outputs and lse
 must be equal bit for bit on either side of that rule: ragged lengths, masks,
@@ -52,6 +52,26 @@ def test_equal_to_the_transposed_tile(library_path, case, acc):
         q, k, v = draw(b, hq, hkv, nq, nk, nq + nk, layout)
         want = Operator(library_path, AttentionConfig(acc=acc, causal=causal, kernel=VT))(q, k, v, return_lse=True)
         got = Operator(library_path, AttentionConfig(acc=acc, causal=causal))(q, k, v, return_lse=True)
+        torch.cuda.synchronize()
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]), (case, acc, layout)
+
+
+# Parts of every length up to past the 64 key blocks, items up to past one
+# round of 256; above 2048 query rows per KV head.
+SPLIT_CASES = [
+    (1, 12, 1, 256, 4099, "bottom_right", 33), (1, 12, 1, 256, 8192, "none", 21), (1, 12, 1, 300, 8321, "bottom_right", 2),
+    (1, 32, 8, 600, 2500, "none", 2), (1, 12, 1, 256, 16640, "none", 2), (1, 12, 1, 256, 2048, "top_left", 22),
+]
+
+
+@pytest.mark.parametrize("case", SPLIT_CASES, ids=str)
+def test_split_equal_to_the_transposed_tile(library_path, case):
+    b, hq, hkv, nq, nk, causal, splits = case
+    for acc, layout in (("fp32", "bhnd"), ("fp16", "bnhd")):
+        say(f"case short split {case} {acc} {layout}")
+        q, k, v = draw(b, hq, hkv, nq, nk, nq + nk, layout)
+        want = Operator(library_path, AttentionConfig(acc=acc, causal=causal, splits=splits, kernel=VT))(q, k, v, return_lse=True)
+        got = Operator(library_path, AttentionConfig(acc=acc, causal=causal, splits=splits))(q, k, v, return_lse=True)
         torch.cuda.synchronize()
         assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]), (case, acc, layout)
 
