@@ -168,8 +168,9 @@ __device__ __forceinline__ T* row_at(T* base, const Strides& st, int b, int h, i
   return base + (int64_t)b * st.b + (int64_t)h * st.h + (int64_t)n * st.n;
 }
 
-// Maximum of two scores. IEEE-754 maximum (NaN-propagating) lowers to a
-// single v_maximum3_f32 with no operand canonicalization; scores are finite.
+// Maximum of two scores or of two parts' lse. IEEE-754 maximum lowers to a
+// single v_maximum3_f32 with no operand canonicalization, and a NaN on either
+// side stays one.
 __device__ __forceinline__ float smax(float a, float b) { return __builtin_elementwise_maximum(a, b); }
 
 // Combine a per-lane value with the lane 32 apart (same query row, other
@@ -358,7 +359,9 @@ __global__ void __launch_bounds__(256) fa_poison_kernel(u32x4* p, uint64_t n16) 
 // the log-sum-exp algebra of the online softmax applied once across parts.
 // A part whose lse is -inf (the row sees none of its keys) has weight 0 (its
 // O row holds zeros); a row that sees no key at all gets O = 0 and
-// lse = -inf. 32 lanes per row: lane i reads the lse of parts i, i + 32, ...,
+// lse = -inf. A part whose lse is NaN (a NaN or an infinity in the row or its
+// keys) makes the row's O and lse NaN, as in a pass over all keys: M is NaN
+// then, and with it every weight but those of parts without keys. 32 lanes per row: lane i reads the lse of parts i, i + 32, ...,
 // so the maximum and the weight sum are reductions over the 32 lanes, and
 // each lane accumulates 4 of the 128 dims over all parts, with the weights
 // broadcast from the lane that computed them and the O loads independent of
@@ -373,7 +376,7 @@ struct CutTiles {
 };
 __device__ __forceinline__ float max32(float x) {
 #pragma unroll
-  for (int m = 16; m >= 1; m >>= 1) x = fmaxf(x, __shfl_xor(x, m, 32));
+  for (int m = 16; m >= 1; m >>= 1) x = smax(x, __shfl_xor(x, m, 32));
   return x;
 }
 __device__ __forceinline__ float sum32(float x) {
@@ -398,7 +401,7 @@ __global__ void __launch_bounds__(256) fa_merge_kernel(const float* __restrict__
       orow = ((int64_t)seq * cut.pack + r % cut.pack) * seq_q + r / cut.pack;
     }
     float mx = -INFINITY;
-    for (int s = sub; s < splits; s += 32) mx = fmaxf(mx, lpart[s * rows + row]);
+    for (int s = sub; s < splits; s += 32) mx = smax(mx, lpart[s * rows + row]);
     mx = max32(mx);
     float a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f, wsum = 0.f;
     if (mx != -INFINITY) {
@@ -430,14 +433,14 @@ __global__ void __launch_bounds__(256) fa_merge_kernel(const float* __restrict__
       }
       wsum = sum32(wsum);
     }
-    const float inv = wsum > 0.f ? 1.f / wsum : 0.f;
+    const float inv = wsum == 0.f ? 0.f : 1.f / wsum;
     const int64_t bh = orow / seq_q;
     const int i = (int)(orow - bh * seq_q);
     const int b = (int)(bh / heads_q), h = (int)(bh - (int64_t)b * heads_q);
     const h4 out = {(_Float16)(a0 * inv), (_Float16)(a1 * inv), (_Float16)(a2 * inv),
                     (_Float16)(a3 * inv)};
     *reinterpret_cast<h4*>(row_at(o, os, b, h, i) + 4 * sub) = out;
-    if (lse && sub == 0) lse[orow] = wsum > 0.f ? mx + __builtin_amdgcn_logf(wsum) * LN2 : -INFINITY;
+    if (lse && sub == 0) lse[orow] = wsum == 0.f ? -INFINITY : mx + __builtin_amdgcn_logf(wsum) * LN2;
   }
 }
 
@@ -463,13 +466,13 @@ __global__ void __launch_bounds__(256) fa_merge_wide_kernel(const float* __restr
   const size_t pstride = (size_t)rows * HD;
   for (int64_t row = blockIdx.x; row < rows; row += gridDim.x) {
     float mx = -INFINITY;
-    for (int s = threadIdx.x; s < splits; s += 32 * G) mx = fmaxf(mx, lpart[s * rows + row]);
+    for (int s = threadIdx.x; s < splits; s += 32 * G) mx = smax(mx, lpart[s * rows + row]);
     mx = max32(mx);
     if (sub == 0) part_m[grp] = mx;
     __syncthreads();
     mx = part_m[0];
 #pragma unroll
-    for (int g = 1; g < G; ++g) mx = fmaxf(mx, part_m[g]);
+    for (int g = 1; g < G; ++g) mx = smax(mx, part_m[g]);
     float a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f, wsum = 0.f;
     if (mx != -INFINITY) {
       const float* col = opart + (size_t)row * HD + 4 * sub;
@@ -513,12 +516,12 @@ __global__ void __launch_bounds__(256) fa_merge_wide_kernel(const float* __restr
         acc += (d & 3) == 0 ? pv.x : (d & 3) == 1 ? pv.y : (d & 3) == 2 ? pv.z : pv.w;
         wall += part_w[g];
       }
-      const float inv = wall > 0.f ? 1.f / wall : 0.f;
+      const float inv = wall == 0.f ? 0.f : 1.f / wall;
       const int64_t bh = row / seq_q;
       const int i = (int)(row - bh * seq_q);
       const int b = (int)(bh / heads_q), h = (int)(bh - (int64_t)b * heads_q);
       row_at(o, os, b, h, i)[d] = (_Float16)(acc * inv);
-      if (lse && d == 0) lse[row] = wall > 0.f ? mx + __builtin_amdgcn_logf(wall) * LN2 : -INFINITY;
+      if (lse && d == 0) lse[row] = wall == 0.f ? -INFINITY : mx + __builtin_amdgcn_logf(wall) * LN2;
     }
     __syncthreads();                        // LDS is reused by the next row
   }
