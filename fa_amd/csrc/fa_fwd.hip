@@ -305,6 +305,14 @@ __device__ __forceinline__ h4 lds_read_tr(const char* p) {
   return __builtin_bit_cast(h4, r);
 }
 
+// Bytes from a head's first K or V row read to the end of its last one, and
+// those of a key block's rows, are below this (validate, check_strides,
+// rows_in_place). It is also the offset of loads that are to fetch nothing:
+// past every buffer's end, and a block's rows on top of it do not wrap to
+// the buffer's start.
+constexpr int64_t kSpanLimit = (int64_t)1 << 31;
+static_assert(kSpanLimit + (kSpanLimit - 1) < (int64_t)1 << 32, "32-bit offsets past the end stay past it");
+
 // Raw-buffer descriptor (gfx9 layout: base address, stride 0, range in
 // bytes, 32-bit data format) for loads from `base`; the hardware returns
 // zeros for any 32-bit word whose offset (per-lane plus scalar) lies at or
@@ -328,7 +336,7 @@ __device__ __forceinline__ i32x4 buffer_rsrc(const void* base, int bytes) {
 // pragma silences that warning for this function alone.
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
-__device__ __forceinline__ void dma_to_lds(i32x4 rsrc, uint32_t lds_addr, int voff, int soff) {
+__device__ __forceinline__ void dma_to_lds(i32x4 rsrc, uint32_t lds_addr, int voff, uint32_t soff) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                :: "s"(lds_addr), "v"(voff), "s"(rsrc), "s"(soff) : "memory", "m0");
 }
@@ -863,23 +871,23 @@ __device__ __forceinline__ void fa_pp_tile(const FaArgs& args, const int tile, c
   // fetches nothing. (Loading the last block again in its place cost 1.5
   // blocks of L2 traffic per tile.)
   const int last = nblk - 1;
-  constexpr int NOWHERE = 0x7ff00000;
-  auto koff = [&](int kb) { return kb <= last ? kb * (BN * krow) : NOWHERE; };
-  auto voff = [&](int vb) { return vb <= last ? vb * (VNAT ? BN * vrow : BN * 2) : NOWHERE; };
+  constexpr uint32_t NOWHERE = (uint32_t)kSpanLimit;
+  auto koff = [&](int kb) { return kb <= last ? (uint32_t)(kb * (BN * krow)) : NOWHERE; };
+  auto voff = [&](int vb) { return vb <= last ? (uint32_t)(vb * (VNAT ? BN * vrow : BN * 2)) : NOWHERE; };
   // DMA instruction m of this wave for the K block at offset ko -> ring slot
   // ks and the V block at offset vo -> slot vs. Branch free: the K/V choice is
   // a select on wave-uniform values; only a wave's last instruction can be
   // absent.
-  auto dma_one = [&](int m, int ko, int ks, int vo, int vs) {
+  auto dma_one = [&](int m, uint32_t ko, int ks, uint32_t vo, int vs) {
     const int q = dw + 4 * m;
     if (m == NIW - 1 && NI % 4 != 0 && q >= NI) return;
     const bool isk = q < KI;
     const int dst = isk ? ks * KBYTES + q * 1024 : NS * KBYTES + vs * VBYTES + (q - KI) * 1024;
-    const int soff = isk ? ko : VNAT ? vo + 4 * (q - KI) * vrow : vo;
+    const uint32_t soff = isk ? ko : VNAT ? vo + (uint32_t)(4 * (q - KI) * vrow) : vo;
     dma_to_lds(isk ? krsrc : vrsrc, lds0 + dst, m < NOFF ? dma_off[m] : vdma, soff);
   };
   auto issue = [&](int kb, int ks, int vb, int vs) {
-    const int ko = koff(kb), vo = voff(vb);
+    const uint32_t ko = koff(kb), vo = voff(vb);
 #pragma unroll
     for (int m = 0; m < NIW; ++m) dma_one(m, ko, ks, vo, vs);
   };
@@ -1004,7 +1012,7 @@ __device__ __forceinline__ void fa_pp_tile(const FaArgs& args, const int tile, c
 #pragma unroll
     for (int i = 0; i < PF; ++i) fr[i] = ld(kb, vb, operand(decltype(kind)::value, i));
   };
-  auto mfma_step = [&](const char* kb, const char* vb, bool with_dma, int dko, int dks, int dvo,
+  auto mfma_step = [&](const char* kb, const char* vb, bool with_dma, uint32_t dko, int dks, uint32_t dvo,
                        int dvs, auto preloaded, auto kind) {
     constexpr int KIND = decltype(kind)::value;
     constexpr int N = KIND == BOTH ? 2 * NQK : NQK;
@@ -1279,7 +1287,8 @@ __device__ __forceinline__ void fa_pp_tile(const FaArgs& args, const int tile, c
       // Pair j + 1's loads, K(j+NS) -> slot sl and V(j+NS-1) -> prev(sl),
       // spread over the step's exponentials (in a burst at its start they
       // measured slower and fetched 4x the bytes from beyond L2).
-      const int ko = koff(j + NS), ks = sl, vo = voff(j + NS - 1), vs = prev(sl);
+      const uint32_t ko = koff(j + NS), vo = voff(j + NS - 1);
+      const int ks = sl, vs = prev(sl);
       valu_step(j * BN, mask, [&](int i) {
         if constexpr (LOADS_IN_VALU) {
 #pragma unroll
@@ -1960,7 +1969,7 @@ int validate(const fa_problem* p, const TileConfig** tile) {
   if (bh >= lim || bh * tiles_q >= lim || p->batch * p->heads_kv >= 65536) return FA_ERR_GEOMETRY;
   // The kernels address a head's contiguous V^T rows, or its contiguous K
   // and V rows (Nk' keys), with 32-bit byte offsets.
-  if ((int64_t)HD * 2 * key_layout(p, *tile).nk_pad >= ((int64_t)1 << 31)) return FA_ERR_GEOMETRY;
+  if ((int64_t)HD * 2 * key_layout(p, *tile).nk_pad >= kSpanLimit) return FA_ERR_GEOMETRY;
   return FA_OK;
 }
 
@@ -2230,7 +2239,7 @@ Strides strides_of(const int64_t* s) { return Strides{s[0], s[1], s[2]}; }
 // (B=8 Hq=64 Hkv=8 Nq=1 Nk=8005: 94 us of copies before a 51 us attention
 // kernel, 147 us per forward; in place 54 us).
 bool rows_in_place(int64_t n, int64_t nk_pad) {
-  const int64_t lim = (int64_t)1 << 30;
+  const int64_t lim = kSpanLimit / (int64_t)sizeof(_Float16);
   return n < lim && n * nk_pad < lim;
 }
 
@@ -2274,7 +2283,7 @@ int check_strides(const fa_problem* p, const fa_strides* s, const KeyLayout& lay
     if (t[2] < HD) return FA_ERR_GEOMETRY;
   if (!lay.pad)
     for (const int64_t* t : {s->k, s->v})
-      if ((t == s->k || lay.vnat) && (p->seq_k - 1) * t[2] * 2 + HD * 2 >= ((int64_t)1 << 31))
+      if ((t == s->k || lay.vnat) && (p->seq_k - 1) * t[2] * 2 + HD * 2 >= kSpanLimit)
         return FA_ERR_GEOMETRY;
   return FA_OK;
 }

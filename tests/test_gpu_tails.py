@@ -60,3 +60,30 @@ def test_far_rows_through_copies_bit_equal(library_path, kernel, rows_apart):
     got = op(q, *far)
     torch.cuda.synchronize()
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("kernel", [3, 4])
+def test_largest_head(library_path, kernel):
+    """8388480 keys, one 128-key block short of the 2 GiB a head's rows may
+    span: offsets of blocks past the last one must not fall into the buffer or
+    wrap. The last key takes half of every row's weight."""
+    nk = (1 << 23) - 128
+    say(f"case largest head kernel={kernel}")
+    g = torch.Generator(device="cuda").manual_seed(kernel)
+    q, k, v = (torch.randn(1, h, n, 128, generator=g, device="cuda", dtype=torch.float16)
+               for h, n in ((2, 1), (1, nk), (1, nk)))
+    q[0, 1] = -q[0, 0]
+    scores = (torch.cat([k[0, 0, i:i + (1 << 20)].float() @ q[0, 0, 0].float()
+                         for i in range(0, nk, 1 << 20)]) * 128 ** -0.5).double()
+    # k_last = a q makes its score a |q|^2 / sqrt(128): as much as all others together.
+    want = torch.logsumexp(scores, 0) * 128 ** 0.5 / (q[0, 0, 0].double() ** 2).sum()
+    k[0, 0, -1] = (want * q[0, 0, 0].double()).half()
+    scores[-1] = (k[0, 0, -1].double() @ q[0, 0, 0].double()) * 128 ** -0.5
+    out, lse = Operator(library_path, AttentionConfig(kernel=kernel, splits=64))(q, k, v, return_lse=True)
+    for h, sign in ((0, 1.0), (1, -1.0)):
+        exact_lse = torch.logsumexp(sign * scores, 0)
+        w = torch.exp(sign * scores - exact_lse)
+        exact = sum(w[i:i + (1 << 20)].float() @ v[0, 0, i:i + (1 << 20)].float()
+                    for i in range(0, nk, 1 << 20))
+        check(out[:, h:h + 1].float().cpu().numpy(), exact.cpu().numpy().reshape(1, 1, 1, 128), "fp32", "largest head")
+        assert abs(float(lse[0, h, 0]) - float(exact_lse)) < 1e-3
