@@ -2009,16 +2009,17 @@ RowLayout row_layout(const fa_problem* p) {
 // Query tiles of one attention launch (one per 256 rows of a row sequence).
 uint64_t grid_size(const fa_problem* p) { return (uint64_t)row_layout(p).tiles(); }
 
-// The few-row kernel (fa_rows_body) runs split launches of the automatic tile
-// choice whose rows fill at most kRowTilesMax of its 32-row tiles per KV head:
-// every tile streams the part's keys for itself, so beyond a few tiles the
-// 256-row tiles, which read them once for eight times the rows, are cheaper.
+// The few-row kernel (fa_rows_body) can run split launches of the automatic
+// tile choice whose rows fill at most kRowTilesMax of its 32-row tiles per KV
+// head, and then does where that is modelled to take no longer than the
+// 256-row tile (choose_few_rows): every row tile streams the part's keys for
+// itself, which a few KV heads leave the bandwidth for and many do not.
 constexpr int64_t kRowTilesMax = 8;
 int64_t row_tiles(const fa_problem* p) {    // 32-row tiles of the launch
   const RowLayout rl = row_layout(p);
   return rl.seqs * ((rl.rows + RT - 1) / RT);
 }
-bool few_rows(const fa_problem* p, int splits) {
+bool few_rows_fit(const fa_problem* p, int splits) {
   const int64_t kv_heads = p->batch * p->heads_kv;
   const int64_t rows = rows_per_kv_head(p);
   return p->kernel == 0 && rows > 0 && rows <= kNaturalVRows &&
@@ -2160,77 +2161,125 @@ double split_cost(const fa_problem* p, const TileConfig* tile, const KeyLayout& 
   return t;
 }
 
-// Modelled duration (us) of a split launch of the few-row kernel with s parts,
-// or, s = 1, of the one-pass kernel in its place. Fitted to part-count sweeps
-// (12 rows behind 4099 to 131072 keys, 192 and 256 rows behind 50001, batches
-// of 64 to 256 tiles): a workgroup's first 256 keys cost 7 us from launch to
-// its result, each further 256 the latency of one block (1.25 us), or, with
-// many workgroups streaming, the time memory (4.7 TB/s over the keys read
-// once) or the L2s (17 TB/s over all of them) take for all workgroups' 128
-// KiB; a CU's later workgroups 5.5 us and their rounds; the merge
-// 3.4 us and 9 ns a part, plus its bytes. The one-pass kernel takes about 1.5
-// us per 128 keys with one wave at work.
-double few_rows_cost(const fa_problem* p, const KeyLayout& lay, int s, int cus) {
-  const double nbt = (double)(lay.nk_pad / 128);
-  const double kv_heads = (double)(p->batch * p->heads_kv);
-  const double round_bytes = 2.0 * 256 * HD * sizeof(_Float16);
-  if (s == 1) {
-    const double tiles = (double)grid_size(p);
-    const double read = std::min(tiles, (double)cus) * kv_heads / tiles * round_bytes / 2 / 4.7e6;
-    return ceil(tiles / cus) * (6.0 + std::max((nbt + 1) * 1.54, nbt * read));
+// Modelled duration (us) of a launch whose rows fit the few-row kernel, with s
+// parts: by that kernel, and by the 256-row natural-V tile (s = 1 is the
+// one-pass forward). Fitted to both kernels over 1 to 256 rows on 1 to 140 KV
+// heads behind 512 to 150000 keys and 1 to 256 parts (720 shapes, 25000
+// timings): the choice it makes there takes 1.3 % longer than the fastest
+// kernel and count timed for a shape, in two of the 720 more than 10 %.
+// A few-row workgroup waits 2.3 us for 256 keys, or as long as memory takes
+// for the active ones' 128 KiB (tiles that read the same keys share part of
+// them), and a die runs its workgroups in rounds of one per CU. A tile waits 2
+// us for 128 keys, 2.5 with rows in both wave groups, or for memory and the
+// matrix units. The last blocks of the longest parts find memory half idle,
+// hence the averages. Both: a fixed part that grows with the rows, and the
+// merge, bound by its bytes or by one row's walk over the parts.
+struct FewRowsModel {
+  double kv_heads, rows, blocks, seen, share;
+  int cus;
+  FewRowsModel(const fa_problem* p, const KeyLayout& lay, int cus) : cus(cus) {
+    kv_heads = (double)(p->batch * p->heads_kv);
+    rows = (double)rows_per_kv_head(p);
+    blocks = (double)(lay.nk_pad / 128);
+    // Key blocks that the last row sees: parts past them are empty.
+    const int64_t keys = p->causal == FA_CAUSAL_TOP_LEFT ? std::min(p->seq_q, p->seq_k) : p->seq_k;
+    seen = (double)((keys + 127) / 128);
+    share = ceil(rows / RT);
   }
-  const double items = (double)row_tiles(p) * s, active = std::min(items, (double)cus);
-  const double share = (double)row_tiles(p) / kv_heads;      // tiles that read the same keys
-  const double rounds = ceil(ceil(nbt / s) / 2);
-  const double per_round =
-      std::max(1.25, std::max(active / share * round_bytes / 4.7e6, active * round_bytes / 17e6));
-  const double rows = (double)(p->batch * p->heads_q) * p->seq_q;
-  return 7.0 + (rounds - 1) * per_round + (ceil(items / cus) - 1) * (5.5 + rounds * per_round) + 3.4 +
-         0.009 * s + rows * s * (HD * 4.0 + 4.0) / 4e6;
+  // Parts with keys that the rows see, and the key blocks of the longest and
+  // of the average one.
+  double parts(int s) const { return ceil(seen * s / blocks); }
+  double longest(int s) const { return std::min(ceil(blocks / s), seen); }
+  double average(int s) const { return std::min(blocks / s, seen); }
+  double merge_us(int s) const {
+    const double all = kv_heads * rows;
+    const int walk = merge_wide((int64_t)all, s) ? (s + 7) / 8 : s;
+    return 4.08 + 0.005 * s + std::max(all * s * (HD * 4.0 + 4.0) / 1.79e6, 0.247 * ((walk + 3) / 4));
+  }
+  double rows_us(int s) const {
+    const double active = std::min(kv_heads * parts(s) * share, (double)cus);
+    const double die = ceil(kv_heads * parts(s) / 8) * share;          // workgroups of a die
+    const double per = std::max(2.25, active / pow(share, 0.615) * (2.0 * 256 * HD * sizeof(_Float16)) / 6.32e6);
+    const double most = ceil(longest(s) / 2), mean = average(s) / 2;
+    return 6.65 + 0.59 * std::min(rows, (double)RT) / RT + (longest(s) > 1 ? 0.68 : 0.0) +
+           (std::max(1.0, mean + 0.58 * (most - mean)) - 1) * per +
+           (ceil(die * 8 / cus) - 1) * (1.6 + most * per) + merge_us(s);
+  }
+  double tile_us(int s) const {
+    const double items = kv_heads * parts(s), active = std::min(items, (double)cus);
+    const double busy = ceil(rows / 32);                               // waves with rows
+    const double per = std::max(rows <= 128 ? 1.98 : 2.52, active * (2.0 * 128 * HD * sizeof(_Float16)) / 6.26e6 +
+                                                               active / cus * 0.506 * busy / 8);
+    const double most = longest(s), mean = average(s);
+    return 6.25 + 0.447 * busy + (std::max(1.0, mean + 0.74 * (most - mean)) - 1) * per +
+           (ceil(items / cus) - 1) * (3.1 + most * per) + (s > 1 ? merge_us(s) : 0.0);
+  }
+};
+
+// How a split launch runs: parts of every tile's keys, and by which kernel.
+struct SplitChoice {
+  int parts = 1;
+  bool few_rows = false;
+};
+
+// The choice for a launch whose rows fit the few-row kernel; requested parts
+// (already clamped) or, 0, those with the shortest modelled launch.
+SplitChoice choose_few_rows(const fa_problem* p, const KeyLayout& lay, int requested, int cus) {
+  const FewRowsModel model(p, lay, cus);
+  SplitChoice best;
+  double best_us = model.tile_us(1);
+  auto consider = [&](int64_t s) {
+    if (s < 2 || s > model.blocks) return;
+    const double r = few_rows_fit(p, (int)s) ? model.rows_us((int)s) : INFINITY, t = model.tile_us((int)s);
+    if (requested || std::min(r, t) < best_us) {
+      best_us = std::min(r, t);
+      best = SplitChoice{(int)s, r <= t};
+    }
+  };
+  if (requested) {
+    consider(requested);
+    return best;
+  }
+  // The counts that change a part's key blocks, in steps of an eighth, and
+  // those that fill the CUs once with parts of either kernel.
+  for (int64_t b = 1; b < model.blocks; b += 1 + b / 8) {
+    const int64_t s = (int64_t)ceil(model.blocks / b);
+    if (s <= kAutoSplitMax) consider(s);
+  }
+  consider(std::min<int64_t>((int64_t)(cus / model.kv_heads), kAutoSplitMax));
+  consider(std::min<int64_t>((int64_t)(floor(cus / 8 / model.share) * 8 / model.kv_heads), kAutoSplitMax));
+  return best;
 }
 
-// Effective split count for a requested one: 0 picks the count with the
-// shortest modelled launch (splitting only when that beats one pass over the
+// How a split launch runs for a requested part count: 0 picks the count with
+// the shortest modelled launch (above the few-row kernel's rows, splitting
+// only when that beats one pass over the
 // keys by 10 %: tiles must leave CUs idle), n >= 1 is clamped to the tile's
-// key blocks (every part then has at least one).
+// key blocks (every part then has at least one). The resolved count requested
+// again resolves to the same choice.
 int resolve_splits(const fa_problem* p, const TileConfig* tile, const KeyLayout& lay,
-                   int requested, int cus, int* out) {
+                   int requested, int cus, SplitChoice* out) {
   if (requested < 0 || requested > kMaxSplits || cus <= 0) return FA_ERR_SPLIT;
   const int64_t nbt = lay.nk_pad / tile->keys;
-  int s = (int)std::min<int64_t>(requested, nbt);
-  if (requested == 0) {
-    s = 1;
-    if (few_rows(p, kAutoSplitMax)) {
-      // The counts that change a workgroup's 256-key rounds, in steps of a quarter.
-      double best = few_rows_cost(p, lay, 1, cus);
-      for (int64_t rounds = 1; 2 * rounds < nbt; rounds += 1 + rounds / 4) {
-        const int64_t n = (nbt + 2 * rounds - 1) / (2 * rounds);
-        if (n > kAutoSplitMax) continue;
-        const double t = few_rows_cost(p, lay, (int)n, cus);
-        if (t < best) {
-          best = t;
-          s = (int)n;
-        }
+  SplitChoice c{(int)std::max<int64_t>(1, std::min<int64_t>(requested, nbt)), false};
+  if (few_rows_fit(p, 2)) {
+    if (requested != 1) c = choose_few_rows(p, lay, requested ? c.parts : 0, cus);
+  } else if (requested == 0 && grid_size(p) < 2 * (uint64_t)cus) {
+    double best = 0.9 * split_cost(p, tile, lay, 1, cus);
+    int most = kAutoSplitMax;
+    if (p->causal != FA_CAUSAL_NONE)
+      most = (int)std::min<int64_t>(
+          most, std::max<int64_t>(16, kAutoCausalItems * cus / (int64_t)grid_size(p)));
+    for (int s = 2; s <= std::min<int64_t>(most, nbt); ++s) {
+      const double t = split_cost(p, tile, lay, s, cus);
+      if (t < best) {
+        best = t;
+        c.parts = s;
       }
-    } else if (grid_size(p) < 2 * (uint64_t)cus) {
-      double best = 0.9 * split_cost(p, tile, lay, 1, cus);
-      auto consider = [&](int c) {
-        if (c > nbt) return;
-        const double t = split_cost(p, tile, lay, c, cus);
-        if (t < best) {
-          best = t;
-          s = c;
-        }
-      };
-      int most = kAutoSplitMax;
-      if (p->causal != FA_CAUSAL_NONE)
-        most = (int)std::min<int64_t>(
-            most, std::max<int64_t>(16, kAutoCausalItems * cus / (int64_t)grid_size(p)));
-      for (int c = 2; c <= most; ++c) consider(c);
     }
   }
-  if ((int64_t)grid_size(p) * s >= ((int64_t)1 << 30)) return FA_ERR_GEOMETRY;
-  *out = std::max(s, 1);
+  if ((int64_t)grid_size(p) * c.parts >= ((int64_t)1 << 30)) return FA_ERR_GEOMETRY;
+  *out = c;
   return FA_OK;
 }
 
@@ -2382,15 +2431,16 @@ int launch(const fa_problem* p, const fa_strides* strides, const void* q, const 
   // The automatic split count depends on the device's CU count; an explicit
   // one does not, so its errors come before any device query.
   int cus = 0;
-  int splits = 1;
+  SplitChoice choice;
   if (ex.split) {
     if (ex.splits == 0) {
       rc = device_cus(&cus);
       if (rc) return rc;
     }
-    rc = resolve_splits(p, tile, lay, ex.splits, cus ? cus : 1, &splits);
+    rc = resolve_splits(p, tile, lay, ex.splits, cus ? cus : 1, &choice);
     if (rc) return rc;
   }
+  const int splits = choice.parts;
   SplitLayout sl = split_layout(p, lay, splits);
   if (!workspace || workspace_bytes < (splits > 1 ? sl.end : lay.workspace_bytes()))
     return FA_ERR_WORKSPACE;
@@ -2416,6 +2466,10 @@ int launch(const fa_problem* p, const fa_strides* strides, const void* q, const 
     rc = device_cus(&cus);
     if (rc) return rc;
   }
+  if (ex.split && ex.splits > 1) {   // its kernel does depend on the device
+    rc = resolve_splits(p, tile, lay, splits, cus, &choice);
+    if (rc) return rc;
+  }
   if (p->kernel == 0 && !lay.vnat) {
     // Both twins are set up by the first call of either: a later call may
     // have to make do without set-up (graph capture).
@@ -2429,7 +2483,7 @@ int launch(const fa_problem* p, const fa_strides* strides, const void* q, const 
       sl = split_layout(p, lay, splits);
     }
   }
-  const bool rows_kernel = splits > 1 && few_rows(p, splits);
+  const bool rows_kernel = choice.few_rows;
   const attn_fn fn = rows_kernel ? kRowsFn[packed][acc] : tile->fn[packed][acc][mode];
   const int lds = rows_kernel ? kRowsLds : tile->lds;
   rc = ensure_lds_limit(fn, lds, rows_kernel ? kNumTiles : (int)(tile - kTiles), packed, acc, mode);
@@ -2703,10 +2757,10 @@ int fa_fwd_split_count(const fa_problem* p, int32_t splits, int32_t cus, int32_t
     rc = device_cus(&n);
     if (rc) return rc;
   }
-  int s = 0;
-  rc = resolve_splits(p, tile, key_layout(p, tile), splits, n, &s);
+  SplitChoice choice;
+  rc = resolve_splits(p, tile, key_layout(p, tile), splits, n, &choice);
   if (rc) return rc;
-  *effective = s;
+  *effective = choice.parts;
   return FA_OK;
 }
 
@@ -2721,9 +2775,10 @@ int fa_fwd_split_workspace_bytes(const fa_problem* p, int32_t splits, uint64_t* 
     rc = device_cus(&cus);
     if (rc) return rc;
   }
-  int s = 0;
-  rc = resolve_splits(p, tile, lay, splits, cus, &s);
+  SplitChoice choice;
+  rc = resolve_splits(p, tile, lay, splits, cus, &choice);
   if (rc) return rc;
+  const int s = choice.parts;
   *bytes = s > 1 ? split_layout(p, lay, s).end : lay.workspace_bytes() + cut_plan(p, tile, lay).bytes();
   return FA_OK;
 }
