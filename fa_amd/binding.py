@@ -361,6 +361,9 @@ class Operator:
             self.check(lib.fa_fwd_workspace_bytes(C.byref(prob), C.byref(size)), "prepare")
         else:
             with torch.cuda.device(q.device):
+                # The automatic count is resolved here, once, and not again by every launch.
+                if splits == 0:
+                    splits = self.split_count(q.shape, k.shape)
                 self.check(lib.fa_fwd_split_workspace_bytes(C.byref(prob), splits,
                                                             C.byref(size)), "prepare")
         p = Plan()

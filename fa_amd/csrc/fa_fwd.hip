@@ -2122,43 +2122,56 @@ constexpr double kMergeLatency = 0.7e-6;
 constexpr int64_t kMergeWideRows = 4096;
 constexpr int kMergeWideParts = 32;
 bool merge_wide(int64_t rows, int splits) { return rows <= kMergeWideRows && splits >= kMergeWideParts; }
-double split_cost(const fa_problem* p, const TileConfig* tile, const KeyLayout& lay, int s, int cus) {
+
+// The model for s = 1..most parts (at most kAutoSplitMax). With a causal mask
+// it sums over a sequence's tiles, each tile for all counts at once: 15 tiles
+// and 125 counts (12 heads, 300 rows, 125 key blocks) take 5 us, where a walk
+// over the tiles for every count took 23, on every automatic launch.
+void split_costs(const fa_problem* p, const TileConfig* tile, const KeyLayout& lay, int cus, int most,
+                 double (&cost)[kAutoSplitMax + 1]) {
   const int bn = tile->keys;
   const int64_t nbt = lay.nk_pad / bn;
   const RowLayout rl = row_layout(p);
   const int64_t nbh = rl.seqs, tiles_q = (rl.rows + kRows - 1) / kRows;
-  const double items = (double)(nbh * tiles_q) * s;
-  double t = 0.0;
   if (p->causal == FA_CAUSAL_NONE) {
-    const double per = (double)((nbt + s - 1) / s) + kItemOverhead;
-    t = ceil(items / cus) * per;
+    for (int s = 1; s <= most; ++s)
+      cost[s] = ceil((double)(nbh * tiles_q) * s / cus) * ((double)((nbt + s - 1) / s) + kItemOverhead);
   } else {
     const int64_t off = p->causal == FA_CAUSAL_BOTTOM_RIGHT ? p->seq_k - p->seq_q : 0;
-    const int64_t len = (nbt + s - 1) / s;                 // longest part
-    double total = 0.0, longest = 0.0, whole = 0.0;
+    // Over the tiles: key blocks seen, parts seen, and parts seen by more than half.
+    int64_t sum = 0, widest = 0;
+    double seen[kAutoSplitMax + 1] = {}, half[kAutoSplitMax + 1] = {};
+    const double eps = 0.25 / (double)nbt;     // vis * s / nbt is a multiple of 1 / nbt
     for (int64_t r = 0; r < tiles_q; ++r) {
       // Keys [0, kend) are seen by the tile's last row (its position + 1):
       // vis key blocks, which fill some parts and reach into one more.
       const int64_t kend = (std::min<int64_t>((r + 1) * kRows, rl.rows) - 1) / rl.pack + 1 + off;
       const int64_t vis = kend <= 0 ? 0 : std::min<int64_t>(nbt, (kend + bn - 1) / bn);
-      const int64_t seen = (vis * s + nbt - 1) / nbt;
-      total += (double)nbh * (vis + seen * kItemOverhead + (s - seen) * kEmptyItem);
-      longest = std::max(longest, std::min(vis, len) + kItemOverhead);
-      whole += (double)(nbh * ((2 * vis * s + nbt - 1) / (2 * nbt)));   // parts seen by more than half
+      if (vis == 0) continue;
+      sum += vis;
+      widest = std::max(widest, vis);
+      const double share = (double)vis / (double)nbt;
+      for (int s = 1; s <= most; ++s) {
+        seen[s] += (double)((int)(share * s - eps) + 1);     // vis * s / nbt rounded up
+        half[s] += (double)(int)(share * s + (0.5 - eps));   // rounded, halves down
+      }
     }
-    t = std::max({total / cus, longest, ceil(whole / cus) * (nbt / s + kItemOverhead)});
+    for (int s = 1; s <= most; ++s) {
+      const double total = (double)nbh * ((double)sum + seen[s] * kItemOverhead +
+                                          ((double)tiles_q * s - seen[s]) * kEmptyItem);
+      const double longest = (double)std::min(widest, (nbt + s - 1) / s) + (widest ? kItemOverhead : 0.0);
+      cost[s] = std::max({total / cus, longest, ceil(nbh * half[s] / cus) * (double)(nbt / s + kItemOverhead)});
+    }
   }
-  if (s > 1) {
-    const double rows = (double)(p->batch * p->heads_q) * p->seq_q;
+  const double rows = (double)(p->batch * p->heads_q) * p->seq_q;
+  for (int s = 2; s <= most; ++s) {
     const double bytes = rows * (s * (HD * 4.0 + 4.0) + HD * 2.0 + 4.0);
     const double block_seconds = bn == 128 ? 3.4e-6 : 1.8e-6;
     // A row's walk: four part loads in flight per lane, over all its parts
     // (fa_merge_kernel) or over an eighth of them (fa_merge_wide_kernel).
     const int walk = merge_wide((int64_t)rows, s) ? (s + 7) / 8 : s;
-    const double merge = std::max(bytes / kMergeBytesPerSecond, ((walk + 3) / 4) * kMergeLatency);
-    t += merge / block_seconds;
+    cost[s] += std::max(bytes / kMergeBytesPerSecond, ((walk + 3) / 4) * kMergeLatency) / block_seconds;
   }
-  return t;
 }
 
 // Modelled duration (us) of a launch whose rows fit the few-row kernel, with s
@@ -2265,18 +2278,19 @@ int resolve_splits(const fa_problem* p, const TileConfig* tile, const KeyLayout&
   if (few_rows_fit(p, 2)) {
     if (requested != 1) c = choose_few_rows(p, lay, requested ? c.parts : 0, cus);
   } else if (requested == 0 && grid_size(p) < 2 * (uint64_t)cus) {
-    double best = 0.9 * split_cost(p, tile, lay, 1, cus);
-    int most = kAutoSplitMax;
+    int64_t most = kAutoSplitMax;
     if (p->causal != FA_CAUSAL_NONE)
-      most = (int)std::min<int64_t>(
-          most, std::max<int64_t>(16, kAutoCausalItems * cus / (int64_t)grid_size(p)));
-    for (int s = 2; s <= std::min<int64_t>(most, nbt); ++s) {
-      const double t = split_cost(p, tile, lay, s, cus);
-      if (t < best) {
-        best = t;
+      most = std::min<int64_t>(
+          most, std::max<int64_t>(16, kAutoCausalItems * (int64_t)cus / (int64_t)grid_size(p)));
+    most = std::min(most, nbt);
+    double cost[kAutoSplitMax + 1];
+    split_costs(p, tile, lay, cus, (int)most, cost);
+    double best = 0.9 * cost[1];
+    for (int s = 2; s <= most; ++s)
+      if (cost[s] < best) {
+        best = cost[s];
         c.parts = s;
       }
-    }
   }
   if ((int64_t)grid_size(p) * c.parts >= ((int64_t)1 << 30)) return FA_ERR_GEOMETRY;
   *out = c;

@@ -10,6 +10,7 @@ last bits, which tells them apart here.
 """
 
 import ctypes as C
+import time
 
 import pytest
 import torch
@@ -79,3 +80,37 @@ def test_kernel_taken(library_path, case, acc):
     torch.cuda.synchronize()
     assert torch.equal(out, again) and torch.equal(lse, lse2), "the resolved count takes another way"
     assert torch.equal(out, want) == (not few_rows)
+
+
+def host_us(fn):
+    """Shortest mean of several short runs: other processes only lengthen one."""
+    def mean():
+        start = time.perf_counter()
+        for _ in range(100):
+            fn()
+        return (time.perf_counter() - start) * 1e4
+
+    return min(mean() for _ in range(20))
+
+
+def test_causal_search_costs_little_more_than_the_unmasked_one(library_path):
+    """300 rows of 12 heads behind 16000 keys: 15 tiles and 125 counts. A walk
+    over the tiles for every count made the search six times the unmasked one."""
+    lib = binding.load_library(library_path)
+    shape = (1, 12, 1, 300, 16000)
+    assert parts(lib, shape, "bottom_right") > 1
+    masked = host_us(lambda: parts(lib, shape, "bottom_right"))
+    unmasked = host_us(lambda: parts(lib, shape))
+    print(f"masked {masked:.1f} us, unmasked {unmasked:.1f} us")
+    assert masked < 3 * unmasked
+
+
+@pytest.mark.gpu
+def test_operator_resolves_the_count_once(library_path):
+    print("case resolved count", flush=True)
+    op = Operator(library_path, AttentionConfig(splits=0, causal="bottom_right"))
+    q = torch.randn(1, 12, 300, 128, device="cuda").half()
+    k = torch.randn(1, 1, 16000, 128, device="cuda").half()
+    op(q, k, k)
+    (plan,) = op.plans.values()
+    assert plan.before[1] == op.split_count(q.shape, k.shape) > 1
