@@ -15,7 +15,9 @@ Mirrors the reference's operator binding
     <status> (<message>)")``;
   * output and workspace tensors are allocated by torch, cached per
     (shapes, device, config), and the same cached output tensor is returned
-    on every call; the workspace grows on demand. Calls of one ``Operator``
+    on every call; the workspace grows on demand. After ``SIGNATURES_KEPT``
+    call signatures the set-up of all of them is dropped, and with it the
+    outputs that nobody else holds. Calls of one ``Operator``
     therefore share its output and workspace: forwards that may overlap on
     different streams need an ``Operator`` each.
 
@@ -25,6 +27,8 @@ construction fails.
 
 import ctypes as C
 import math
+import struct
+import weakref
 from dataclasses import dataclass
 
 FA_ACC = {"fp32": 0, "fp16": 1}
@@ -161,6 +165,11 @@ LAYOUT_ERROR = ("Q/K/V must be [B,H,N,128] views with a contiguous last dimensio
 # Query rows per attention tile.
 TILE_ROWS = 256
 
+# Call signatures an Operator keeps set up. A decode loop has a new one (one
+# more key) in every step, so there has to be a limit; a program's recurring
+# ones are far fewer.
+SIGNATURES_KEPT = 64
+
 
 def query_tiles(batch, heads_q, heads_kv, seq_q):
     """Attention tiles of one launch, as the library lays them out: unpacked,
@@ -202,10 +211,14 @@ class Operator:
         self.config = config
         self.lib = load_library(library) if not isinstance(library, C.CDLL) else library
         self.workspace = None
-        self.buffers = {}
         self.plans = {}          # call signature -> Plan
+        # The outputs of the plans, and those of dropped plans that the caller
+        # still holds: a signature met again gets the same tensor, and no two
+        # live outputs of different shapes share memory.
+        self.buffers = weakref.WeakValueDictionary()
+        self.captured = {}       # plans and workspaces that captured graphs refer to
         self.streams = {}        # (device index, raw stream) -> torch stream
-        self.tiles = {}          # (q shape, k shape) -> (rows, keys) granularity
+        self.tiles = {}          # selector -> (rows, keys) granularity
         self.last = None
 
     def message(self, status):
@@ -217,14 +230,15 @@ class Operator:
             raise RuntimeError(f"fa_fwd {where}: {status} ({self.message(status)})")
 
     def tile(self, q_shape, k_shape):
-        """(query rows, keys) granularity of the kernel the library would use."""
-        key = (tuple(q_shape), tuple(k_shape))
-        if key not in self.tiles:
+        """(query rows, keys) granularity of the kernel the library would use.
+        Every tile masks ragged tails, so it follows from the selector alone."""
+        kernel = self.config.kernel
+        if kernel not in self.tiles:
             prob = make_problem(q_shape, k_shape, 1.0, self.config)
             rows, keys = C.c_int32(), C.c_int32()
             self.check(self.lib.fa_fwd_tile(C.byref(prob), C.byref(rows), C.byref(keys)), "tile")
-            self.tiles[key] = (rows.value, keys.value)
-        return self.tiles[key]
+            self.tiles[kernel] = (rows.value, keys.value)
+        return self.tiles[kernel]
 
     def kernel(self, q_shape, k_shape):
         """1-based tile configuration the library would launch (automatic choice resolved)."""
@@ -241,7 +255,9 @@ class Operator:
         (``config.splits`` resolved; ``cus`` = 0: the current device)."""
         if self.config.splits is None:
             return 1
-        prob = make_problem(q_shape, k_shape, 1.0, self.config)
+        return self.problem_splits(make_problem(q_shape, k_shape, 1.0, self.config), cus)
+
+    def problem_splits(self, prob, cus=0):
         n = C.c_int32()
         self.check(self.lib.fa_fwd_split_count(C.byref(prob), self.config.splits, cus,
                                                C.byref(n)), "split")
@@ -259,24 +275,27 @@ class Operator:
         rows, keys = self.tile(q.shape, k.shape)
         if nq % rows or k.shape[2] % keys or max(nq, k.shape[2]) >= 2 ** 30:
             raise ValueError(f"unsupported query/key tail (Nq % {rows}, Nk % {keys})")
+        device = q.device
+        if device.type != "cuda" or k.device != device or v.device != device \
+                or not q.dtype == k.dtype == v.dtype == torch.float16:
+            raise ValueError("Q/K/V must be FP16 on the same GPU")
         for t in (q, k, v):
-            if t.device.type != "cuda" or t.device != q.device or t.dtype != torch.float16:
-                raise ValueError("Q/K/V must be FP16 on the same GPU")
-            st = t.stride()
-            if st[3] != 1 or any(x % 8 or x < 0 for x in st[:3]) or st[2] < 128 \
-                    or t.data_ptr() % 16:
+            b, h, n, d = t.stride()
+            if d != 1 or b % 8 or h % 8 or n % 8 or b < 0 or h < 0 or n < 128 or t.data_ptr() % 16:
                 raise ValueError(LAYOUT_ERROR)
 
     def buffers_for(self, q, k, lse=False):
         import torch
 
-        key = (tuple(q.shape), tuple(k.shape), q.device, self.config, lse)
-        if key not in self.buffers:
+        key = (q.shape, k.shape, q.device, self.config, lse)
+        out = self.buffers.get(key)
+        if out is None:
             if lse:
-                self.buffers[key] = torch.empty(q.shape[:3], dtype=torch.float32, device=q.device)
+                out = torch.empty(q.shape[:3], dtype=torch.float32, device=q.device)
             else:
-                self.buffers[key] = torch.empty(q.shape, dtype=torch.float16, device=q.device)
-        return self.buffers[key]
+                out = torch.empty(q.shape, dtype=torch.float16, device=q.device)
+            self.buffers[key] = out
+        return out
 
     # Capture buffers are for small debug inputs, as in the reference binding
     # (binding.py:40-42: at most 64 Mi FP32 values).
@@ -285,29 +304,30 @@ class Operator:
     def stats_for(self, q, k, prob):
         import torch
 
-        key = (tuple(q.shape), tuple(k.shape), q.device, self.config, "stats")
-        if key not in self.buffers:
-            count, block = C.c_uint64(), C.c_int32()
-            self.check(self.lib.fa_fwd_capture_count(C.byref(prob), C.byref(count),
-                                                     C.byref(block)), "capture")
-            if count.value > self.CAPTURE_LIMIT:
-                raise ValueError("debug capture is restricted to small inputs (at most 256 MiB)")
+        count, block = C.c_uint64(), C.c_int32()
+        self.check(self.lib.fa_fwd_capture_count(C.byref(prob), C.byref(count), C.byref(block)),
+                   "capture")
+        if count.value > self.CAPTURE_LIMIT:
+            raise ValueError("debug capture is restricted to small inputs (at most 256 MiB)")
+        key = (q.shape, k.shape, q.device, self.config, "stats")
+        stats = self.buffers.get(key)
+        if stats is None:
             nblk = count.value // (4 * q.shape[0] * q.shape[1] * q.shape[2])
-            stats = torch.empty((4, nblk) + tuple(q.shape[:3]), dtype=torch.float32,
-                                device=q.device)
-            self.buffers[key] = (stats, block.value)
-        return self.buffers[key]
+            stats = self.buffers[key] = torch.empty((4, nblk) + tuple(q.shape[:3]),
+                                                    dtype=torch.float32, device=q.device)
+        return stats, block.value
 
     def trace_for(self, q, k, prob):
         import torch
 
-        key = (tuple(q.shape), tuple(k.shape), q.device, self.config, "trace")
-        if key not in self.buffers:
+        key = (q.shape, k.shape, q.device, self.config, "trace")
+        trace = self.buffers.get(key)
+        if trace is None:
             count = C.c_uint64()
             self.check(self.lib.fa_fwd_trace_count(C.byref(prob), C.byref(count)), "trace")
-            self.buffers[key] = torch.empty((count.value // TRACE_WORDS, TRACE_WORDS),
-                                            dtype=torch.int64, device=q.device)
-        return self.buffers[key]
+            trace = self.buffers[key] = torch.empty((count.value // TRACE_WORDS, TRACE_WORDS),
+                                                    dtype=torch.int64, device=q.device)
+        return trace
 
     def __call__(self, q, k, v, scale=None, return_lse=False):
         """O (cached tensor), or (O, lse) with ``return_lse``: lse [B, Hq, Nq] FP32
@@ -323,16 +343,21 @@ class Operator:
 
         # Everything but the pointers' alignment follows from these values,
         # so one lookup stands for the checks and the set-up of a signature
-        # met before: a call's host time is 12 us of which the launches are 6
-        # (24 us with every check and conversion made anew), which is what
-        # bounds a short decode step.
+        # met before. A decode step of 12 heads (two launches, 7 us of the
+        # host's time) takes 13.5 us where its signature is met again, and
+        # 28.6 where its key length is new, as in a decode loop, both with the
+        # slicing of the cache; 25.6 and 34.7 with every check, conversion and
+        # allocation made anew each time.
         if scale is not None:
             scale = float(scale)
         key = (q.shape, k.shape, v.shape, q.stride(), k.stride(), v.stride(), q.dtype, k.dtype,
                v.dtype, q.device, k.device, v.device, scale, bool(return_lse))
         plan = self.plans.get(key)
         if plan is None or plan.config is not self.config:
-            plan = self.plans[key] = self.plan(q, k, v, scale, return_lse)
+            plan = self.plan(q, k, v, scale, return_lse)
+            if len(self.plans) >= SIGNATURES_KEPT:
+                self.plans.clear()
+            self.plans[key] = plan
         qp, kp, vp = q.data_ptr(), k.data_ptr(), v.data_ptr()
         if (qp | kp | vp) % 16:
             raise ValueError(LAYOUT_ERROR)
@@ -363,7 +388,7 @@ class Operator:
             with torch.cuda.device(q.device):
                 # The automatic count is resolved here, once, and not again by every launch.
                 if splits == 0:
-                    splits = self.split_count(q.shape, k.shape)
+                    splits = self.problem_splits(prob)
                 self.check(lib.fa_fwd_split_workspace_bytes(C.byref(prob), splits,
                                                             C.byref(size)), "prepare")
         p = Plan()
@@ -378,10 +403,8 @@ class Operator:
             raise ValueError("capture, trace and sync modes need contiguous Q/K/V")
         st = None
         if strided:
-            st = FaStrides()
-            for name, t in (("q", q), ("k", k), ("v", v), ("o", p.out)):
-                getattr(st, name)[:] = t.stride()[:3]
-            st = C.byref(st)
+            st = C.byref(FaStrides.from_buffer_copy(struct.pack(
+                "=12q", *q.stride()[:3], *k.stride()[:3], *v.stride()[:3], *p.out.stride()[:3])))
         # The call is fn(*before, q, k, v, *outputs, *after, workspace, bytes, stream);
         # an output of None is passed as a null pointer.
         p.before, p.outputs, p.after = (C.byref(prob),), (p.out, p.lse), ()
@@ -417,6 +440,8 @@ class Operator:
             if len(self.streams) >= 64:
                 self.streams.clear()
             stream = self.streams[index, raw] = torch.cuda.current_stream(index)
+        if raw and torch.cuda.is_current_stream_capturing():   # never the default stream
+            self.captured[id(plan), ws.data_ptr()] = plan, ws
         outputs = [t.data_ptr() if t is not None else None for t in plan.outputs]
         status = plan.fn(*plan.before, qp, kp, vp, *outputs, *plan.after, ws.data_ptr(), ws.numel(),
                          raw)
