@@ -30,28 +30,35 @@ def make(b, hq, hkv, nq, nk, seed, sig=1.0):
     return q, k, v
 
 
-# (B, Hq, Hkv, Nq, Nk, causal, splits)
+# (B, Hq, Hkv, Nq, Nk, causal, splits, few-row kernel): short parts of few rows
+# run on the 256-row tile, which is then the faster one. None: the rows see one
+# block of 32 keys, where both kernels may give the same bits.
 CASES = [
-    (1, 12, 1, 1, 129, "none", 2),            # two blocks in all, one key in the last
-    (1, 12, 1, 1, 4099, "none", 0),
-    (2, 8, 2, 8, 1000, "none", 3),            # 32 packed rows: one full tile
-    (2, 8, 2, 8, 1000, "top_left", 3),        # only the first 8 keys are seen
-    (1, 3, 1, 11, 2048, "bottom_right", 5),   # 33 rows: a tile of one row
-    (1, 1, 1, 31, 777, "bottom_right", 7),
-    (3, 4, 4, 1, 515, "none", 2),             # no shared KV heads
-    (1, 12, 1, 16, 5001, "bottom_right", 0),  # 192 rows, 6 tiles
-    (1, 8, 1, 32, 3000, "none", 11),          # 256 rows, the most it takes
-    (1, 1, 1, 257, 3000, "none", 4),          # one more
-    (1, 2, 1, 128, 64 * 128, "bottom_right", 64),
-    (2, 2, 1, 70, 300, "bottom_right", 3),
-    (1, 2, 2, 200, 130, "bottom_right", 2),   # rows 0..69 see no key
+    (1, 12, 1, 1, 129, "none", 2, False),           # two blocks in all, one key in the last
+    (1, 12, 1, 8, 129, "none", 2, True),
+    (1, 12, 1, 1, 4099, "none", 0, False),
+    (1, 12, 1, 1, 4099, "none", 17, True),
+    (2, 8, 2, 8, 1000, "none", 3, True),            # 32 packed rows: one full tile
+    (2, 8, 2, 8, 1000, "top_left", 3, None),        # only the first 8 keys are seen
+    (2, 16, 2, 16, 1000, "top_left", 3, None),      # the first 16, by 128 rows
+    (1, 3, 1, 11, 2048, "bottom_right", 5, True),   # 33 rows: a tile of one row
+    (1, 1, 1, 31, 777, "bottom_right", 7, False),
+    (1, 1, 1, 31, 777, "bottom_right", 3, True),
+    (3, 4, 4, 1, 515, "none", 2, True),             # no shared KV heads
+    (1, 12, 1, 16, 5001, "bottom_right", 0, True),  # 192 rows, 6 tiles
+    (1, 8, 1, 32, 3000, "none", 11, True),          # 256 rows, the most it takes
+    (1, 1, 1, 257, 3000, "none", 4, False),         # one more
+    (1, 2, 1, 128, 64 * 128, "bottom_right", 64, False),
+    (1, 2, 1, 128, 64 * 128, "bottom_right", 30, True),
+    (2, 2, 1, 70, 300, "bottom_right", 3, True),
+    (1, 2, 2, 200, 130, "bottom_right", 2, True),   # rows 0..69 see no key
 ]
 
 
 @pytest.mark.parametrize("layout", ["bhnd", "bnhd"])
 @pytest.mark.parametrize("acc", ["fp32", "fp16"])
-@pytest.mark.parametrize("b,hq,hkv,nq,nk,causal,splits", CASES)
-def test_few_rows_vs_f64(library_path, b, hq, hkv, nq, nk, causal, splits, acc, layout):
+@pytest.mark.parametrize("b,hq,hkv,nq,nk,causal,splits,few_rows", CASES)
+def test_few_rows_vs_f64(library_path, b, hq, hkv, nq, nk, causal, splits, few_rows, acc, layout):
     say(f"case few rows B{b} Hq{hq} Hkv{hkv} nq={nq} nk={nk} causal={causal} splits={splits} "
         f"acc={acc} {layout}")
     q, k, v = make(b, hq, hkv, nq, nk, seed=nq * 31 + nk)
@@ -74,6 +81,10 @@ def test_few_rows_vs_f64(library_path, b, hq, hkv, nq, nk, causal, splits, acc, 
     check_lse(lse.cpu().numpy(), exact_lse, "few rows")
     empty = np.isneginf(exact_lse)
     assert bool(np.all(out[empty] == 0)), "rows without keys must be exactly zero"
+    # The kernels round P against other running maxima: other bits, another kernel.
+    tile = AttentionConfig(acc=acc, causal=causal, splits=op.split_count(q.shape, k.shape), kernel=4)
+    same = np.array_equal(out, Operator(library_path, tile)(*dev).float().cpu().numpy())
+    assert few_rows is None or same != few_rows
 
 
 @pytest.mark.parametrize("acc", ["fp32", "fp16"])
@@ -91,13 +102,14 @@ def test_few_rows_stress_and_repeat(library_path, acc):
     check_lse(lse.cpu().numpy(), orc.lse_f64(q, k), "few rows stress")
 
 
+@pytest.mark.parametrize("heads", [4, 48])        # the 256-row tile, the few-row kernel
 @pytest.mark.parametrize("rows_apart", [(1 << 22) - 8, 1 << 22])
-def test_few_rows_far_apart(library_path, rows_apart):
+def test_few_rows_far_apart(library_path, rows_apart, heads):
     """130 keys 2^22 elements apart are copied (256 padded rows span 2 GiB),
     8 elements closer they are read in place: the same output bit for bit."""
     nk = 130
-    say(f"case few rows far apart n={rows_apart}")
-    q, k, v = (t.cuda() for t in make(1, 4, 1, 2, nk, seed=9))
+    say(f"case few rows far apart n={rows_apart} heads={heads}")
+    q, k, v = (t.cuda() for t in make(1, heads, 1, 2, nk, seed=9))
     op = Operator(library_path, AttentionConfig(splits=2))
     want = op(q, k, v).clone()
     far = []
