@@ -177,7 +177,7 @@ def query_tiles(batch, heads_q, heads_kv, seq_q):
     that needs fewer 256-row tiles (grouped-query attention with few query
     rows), ``batch * heads_kv`` sequences of ``seq_q * group`` rows, the
     group's query heads position by position. Every row's result is the same
-    either way. (One trace record per tile: ``fa_fwd_trace_count`` / 8.)"""
+    either way, but for tiles cut into key parts. (One trace record per tile: ``fa_fwd_trace_count`` / 8.)"""
     def tiles(seqs, rows):
         return seqs * -(-rows // TILE_ROWS)
 

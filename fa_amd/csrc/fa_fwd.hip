@@ -5,7 +5,7 @@
 // = head / group, backends/cce_fa_nk_nz_vector_fp32_v5_sumpack/project/
 // op_kernel/panel_kernel.h:264-274): a query tile is BM = 256 query rows of
 // one (batch, head), 8 waves x 32 rows. The attention kernel is persistent:
-// one workgroup per CU takes tiles from a counter until none are left. For a
+// one workgroup per CU takes tiles from work queues until none are left. For a
 // tile it streams the whole key range in blocks of BN keys; each K block and
 // V block is staged once in LDS (a ring of slots) and read by every wave,
 // and every wave keeps its Q fragments, O accumulators and softmax
@@ -13,9 +13,10 @@
 // are masked, the per-row log-sum-exp is written on request, and an optional
 // causal mask makes a tile stream only the key blocks up to its diagonal.
 // Separate instantiations add the capture (per-block softmax statistics),
-// trace (per-tile clock stamps) and synchronous debug modes, and the
-// key-split mode: work items are (tile, part of its key range), whose
-// partial results a merge kernel combines through their log-sum-exp.
+// trace (per-tile clock stamps) and synchronous debug modes, and parts: work
+// items that are a part of a tile's key range, of every tile (key split) or of
+// the last ones, whose results a merge kernel combines through their
+// log-sum-exp. Key splits of few rows have a kernel of their own too.
 //
 // Matrix products run transposed so the softmax is lane-local:
 //   S^T = K Q^T   v_mfma_f32_32x32x16_f16, A = K rows from LDS, B = Q^T
@@ -258,7 +259,7 @@ __global__ void __launch_bounds__(256) fa_prep_kernel(const _Float16* __restrict
 }
 
 // Prep for the tile that reads V in its natural layout: resets the attention
-// kernel's tile counter and, for a K or V whose rows lie too far apart for
+// kernel's work queues and, for a K or V whose rows lie too far apart for
 // 32-bit offsets (kpad non-null, see rows_in_place), writes zero-padded
 // copies of both: kpad[kv][key] and vpad[kv][key] hold the
 // caller's rows for keys below nk_valid and zeros up to nk_pad, one 64-key
@@ -1522,8 +1523,9 @@ __device__ __forceinline__ void fa_pp_body(const FaArgs& args) {
   }
 }
 
-// The few-row kernel: split mode for row sequences that fill at most
-// kRowTilesMax 32-row tiles per KV head (decode, a few tokens behind a cache).
+// The few-row kernel: key splits of row sequences that fill at most
+// kRowTilesMax 32-row tiles per KV head (decode, a few tokens behind a cache),
+// where it is modelled to be no slower than the 256-row tile.
 // There the forward reads every key once and is bound by that read, so the
 // kernel is laid out for bytes in flight and no waiting: a work item is one
 // tile of 32 rows and one part of its keys, and each of the 8 waves takes
@@ -1991,7 +1993,8 @@ uint64_t capture_count(const fa_problem* p, const TileConfig* tile, const KeyLay
 // sequences of Nq * group rows (the group's query heads position by
 // position), taken whenever that needs fewer 256-row tiles: grouped-query
 // attention with fewer than 256 query rows per head, or ragged tails that
-// pack tighter. Both give every row the same result bit for bit.
+// pack tighter. Both give every row of an uncut tile the same result bit for
+// bit (which tiles a launch cuts follows from their number, see cut_plan).
 struct RowLayout {
   int64_t seqs;   // sequences
   int64_t rows;   // rows per sequence
@@ -2504,7 +2507,7 @@ int launch(const fa_problem* p, const fa_strides* strides, const void* q, const 
   if (rc) return rc;
 
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  // Workspace: [V^T] [padded K] [padded V] counter, as the layout has them.
+  // Workspace: [V^T] [padded K] [padded V] work queues, as the layout has them.
   const bool copies = lay.pad && !(rows_in_place(ks.n, lay.nk_pad) &&
                                    (!lay.vnat || rows_in_place(vs.n, lay.nk_pad)));
   _Float16* ws = static_cast<_Float16*>(workspace);
@@ -2539,7 +2542,7 @@ int launch(const fa_problem* p, const fa_strides* strides, const void* q, const 
     void* pad_args[] = {&kk, &vv, &kpad, &vpad, &nk_valid, &nk_pad, &heads_kv, &ks, &vs, &next_tile};
     const dim3 groups((unsigned)(lay.nk_pad / PAD_GROUP), (unsigned)(p->batch * p->heads_kv));
     // The natural-V tile without copies needs the pad kernel only for
-    // the counter, which a launch of at most one work item per CU does not
+    // the work queues, which a launch of at most one work item per CU does not
     // use (fa_pp_body): then nothing runs before the attention kernel.
     bool ok = true;
     if (!lay.vnat)

@@ -18,8 +18,10 @@
  * tiles (grouped-query attention with few query rows per head, e.g. decode)
  * -- the Nq * (Hq / Hkv) rows of one (b, KV head) in position-major order
  * (row r is position r / group of query head hkv * group + r % group). A
- * row's result is the same bit for bit either way; packing only lets the
- * heads that share K and V share a tile.
+ * row's result is the same bit for bit either way, as long as neither tile is
+ * cut into key parts (see fa_fwd(): packing changes the number of tiles, and
+ * with it which ones are cut); packing only lets the heads that share K and V
+ * share a tile.
  *
  * V layouts: the 128-key tile comes in two forms with identical results bit
  * for bit. pp_n128_r2 (and the 64-key tiles) read V^T, a key-permuted
@@ -147,9 +149,10 @@ int fa_fwd_workspace_bytes(const fa_problem* p, uint64_t* bytes);
  * multiple of 256, may cut the tiles of its last, partial round (tile count
  * modulo 256, the last ones) into parts of their key range, so that they
  * occupy every CU, and combine the parts as fa_fwd_split() does: those rows
- * then differ from an uncut launch's by FP32 summation order. This is a
- * function of the problem alone; with a workspace that holds all else but
- * not the parts, nothing is cut.
+ * then differ from an uncut launch's by FP32 summation order. Whether and
+ * where tiles are cut depends on the problem and the workspace size alone: in
+ * a workspace of fa_fwd_workspace_bytes(p) or more they are, in one that holds
+ * all else but not the parts nothing is. fa_fwd_capture() cuts nothing.
  */
 int fa_fwd(const fa_problem* p, const void* q, const void* k, const void* v, void* o,
            void* workspace, uint64_t workspace_bytes, void* stream);
@@ -290,7 +293,7 @@ const char* fa_kernel_name(int32_t kernel);
  * fa_fwd() without a caller workspace, for callers that cannot allocate
  * device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc). No counterpart in the reference. The
- * workspace (fa_fwd_workspace_bytes(): the tile counter, V^T for the V^T
+ * workspace (fa_fwd_workspace_bytes(): the work queues, V^T for the V^T
  * tiles, the room for a ragged key tail's copies) lives in a static device array
  * of FA_NOALLOC_SCRATCH_BYTES per GPU, which the library holds from module
  * load until the process ends; problems whose fa_fwd_workspace_bytes()
@@ -326,7 +329,10 @@ int fa_fwd_noalloc(const fa_problem* p, const void* q, const void* k, const void
  * lse = M + ln sum_s exp(lse_s - M). For problems with fewer query tiles
  * than the GPU has CUs (short query ranges, small batch against long keys)
  * this keeps every CU busy; fa_fwd() runs one work item per tile and leaves
- * the rest idle. The results equal fa_fwd_lse()'s up to FP32 summation order
+ * the rest idle. Launches of at most 256 rows per KV head run, with the
+ * automatic tile, a kernel for few rows in place of the 256-row tile where that
+ * is modelled to take no longer with the part count at hand.
+ * The results equal fa_fwd_lse()'s up to FP32 summation order
  * (FP16 accumulator: each part rounds its own 512-key packets). splits = 0
  * picks the count automatically on the current device (fa_fwd_split_count),
  * n >= 1 is clamped to the key blocks of the tile, and a count of 1 is
@@ -347,7 +353,9 @@ int fa_fwd_split(const fa_problem* p, int32_t splits, const fa_strides* strides,
  * to 256 (work items per CU, per-item overhead, the merge's HBM traffic or,
  * with few rows, its walk over the parts; for at most 4096 rows and 32 parts
  * or more the merge gives each row a workgroup) and splits only when that
- * beats one pass over the keys by 10 %. */
+ * beats one pass over the keys by 10 %; for at most 256 rows per KV head it
+ * compares the counts of both kernels (see above) with one pass. The count
+ * returned, requested again, runs the same launch without the search. */
 
 /* Static message for a status code. */
 const char* fa_strerror(int status);
