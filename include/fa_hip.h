@@ -149,7 +149,8 @@ int fa_fwd_workspace_bytes(const fa_problem* p, uint64_t* bytes);
  * multiple of 256, may cut the tiles of its last, partial round (tile count
  * modulo 256, the last ones) into parts of their key range, so that they
  * occupy every CU, and combine the parts as fa_fwd_split() does: those rows
- * then differ from an uncut launch's by FP32 summation order. Whether and
+ * then differ from an uncut launch's by FP32 summation order (FP16
+ * accumulator: and by where its 512-key packets start). Whether and
  * where tiles are cut depends on the problem and the workspace size alone: in
  * a workspace of fa_fwd_workspace_bytes(p) or more they are, in one that holds
  * all else but not the parts nothing is. fa_fwd_capture() cuts nothing.
