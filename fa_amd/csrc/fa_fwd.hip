@@ -990,7 +990,7 @@ __device__ __forceinline__ void fa_pp_tile(const FaArgs& args, const int tile, c
   // the PV half (KIND; with both halves in each, a tile's MFMAs took two half
   // steps on each group more: a batch of 4 x 32 heads over 2048 keys, 2 to 16
   // blocks a tile, 182 us instead of 180; 1000 causal rows, 8 blocks, 31.4
-  // instead of 30.0; 256 blocks a tile 2 % more).
+  // instead of 30.0; no difference at 256 blocks a tile).
   // Operand i of a step: QK op n = i / 2 (even i) covers S tile n % KT at
   // k-step n / KT, so consecutive QK ops alternate accumulators; with PV ops
   // in between, no accumulator is reused within four MFMAs and dependent
