@@ -212,10 +212,10 @@ class Operator:
         self.lib = load_library(library) if not isinstance(library, C.CDLL) else library
         self.workspace = None
         self.plans = {}          # call signature -> Plan
-        # The outputs of the plans, and those of dropped plans that the caller
-        # still holds: a signature met again gets the same tensor, and no two
-        # live outputs of different shapes share memory.
-        self.buffers = weakref.WeakValueDictionary()
+        # Weak references to the outputs of the plans, and to those of dropped
+        # plans that the caller still holds: a signature met again gets the same
+        # tensor, and no two live outputs of different shapes share memory.
+        self.buffers = {}
         self.captured = {}       # plans and workspaces that captured graphs refer to
         self.streams = {}        # (device index, raw stream) -> torch stream
         self.tiles = {}          # selector -> (rows, keys) granularity
@@ -284,18 +284,31 @@ class Operator:
             if d != 1 or b % 8 or h % 8 or n % 8 or b < 0 or h < 0 or n < 128 or t.data_ptr() % 16:
                 raise ValueError(LAYOUT_ERROR)
 
+    def buffer(self, q, k, what, make):
+        """The live buffer `what` of these shapes, or a new one from make()."""
+        key = (q.shape, k.shape, q.device, self.config, what)
+        held = self.buffers.get(key)
+        tensor = held() if held is not None else None
+        if tensor is None:
+            tensor = make()
+            self.buffers[key] = weakref.ref(tensor)
+        return tensor
+
     def buffers_for(self, q, k, lse=False):
         import torch
 
-        key = (q.shape, k.shape, q.device, self.config, lse)
-        out = self.buffers.get(key)
-        if out is None:
-            if lse:
-                out = torch.empty(q.shape[:3], dtype=torch.float32, device=q.device)
-            else:
-                out = torch.empty(q.shape, dtype=torch.float16, device=q.device)
-            self.buffers[key] = out
-        return out
+        if lse:
+            return self.buffer(q, k, True, lambda: torch.empty(
+                q.shape[:3], dtype=torch.float32, device=q.device))
+        return self.buffer(q, k, False, lambda: torch.empty(
+            q.shape, dtype=torch.float16, device=q.device))
+
+    def drop_plans(self):
+        """Forgets the plans, and every buffer that nobody else holds."""
+        self.plans.clear()
+        for key, held in list(self.buffers.items()):
+            if held() is None:
+                self.buffers.pop(key, None)
 
     # Capture buffers are for small debug inputs, as in the reference binding
     # (binding.py:40-42: at most 64 Mi FP32 values).
@@ -309,25 +322,18 @@ class Operator:
                    "capture")
         if count.value > self.CAPTURE_LIMIT:
             raise ValueError("debug capture is restricted to small inputs (at most 256 MiB)")
-        key = (q.shape, k.shape, q.device, self.config, "stats")
-        stats = self.buffers.get(key)
-        if stats is None:
-            nblk = count.value // (4 * q.shape[0] * q.shape[1] * q.shape[2])
-            stats = self.buffers[key] = torch.empty((4, nblk) + tuple(q.shape[:3]),
-                                                    dtype=torch.float32, device=q.device)
+        nblk = count.value // (4 * q.shape[0] * q.shape[1] * q.shape[2])
+        stats = self.buffer(q, k, "stats", lambda: torch.empty(
+            (4, nblk) + tuple(q.shape[:3]), dtype=torch.float32, device=q.device))
         return stats, block.value
 
     def trace_for(self, q, k, prob):
         import torch
 
-        key = (q.shape, k.shape, q.device, self.config, "trace")
-        trace = self.buffers.get(key)
-        if trace is None:
-            count = C.c_uint64()
-            self.check(self.lib.fa_fwd_trace_count(C.byref(prob), C.byref(count)), "trace")
-            trace = self.buffers[key] = torch.empty((count.value // TRACE_WORDS, TRACE_WORDS),
-                                                    dtype=torch.int64, device=q.device)
-        return trace
+        count = C.c_uint64()
+        self.check(self.lib.fa_fwd_trace_count(C.byref(prob), C.byref(count)), "trace")
+        return self.buffer(q, k, "trace", lambda: torch.empty(
+            (count.value // TRACE_WORDS, TRACE_WORDS), dtype=torch.int64, device=q.device))
 
     def __call__(self, q, k, v, scale=None, return_lse=False):
         """O (cached tensor), or (O, lse) with ``return_lse``: lse [B, Hq, Nq] FP32
@@ -344,8 +350,8 @@ class Operator:
         # Everything but the pointers' alignment follows from these values,
         # so one lookup stands for the checks and the set-up of a signature
         # met before. A decode step of 12 heads (two launches, 7 us of the
-        # host's time) takes 13.5 us where its signature is met again, and
-        # 28.6 where its key length is new, as in a decode loop, both with the
+        # host's time) takes 13.3 us where its signature is met again, and
+        # 27.9 where its key length is new, as in a decode loop, both with the
         # slicing of the cache; 25.6 and 34.7 with every check, conversion and
         # allocation made anew each time.
         if scale is not None:
@@ -356,7 +362,7 @@ class Operator:
         if plan is None or plan.config is not self.config:
             plan = self.plan(q, k, v, scale, return_lse)
             if len(self.plans) >= SIGNATURES_KEPT:
-                self.plans.clear()
+                self.drop_plans()
             self.plans[key] = plan
         qp, kp, vp = q.data_ptr(), k.data_ptr(), v.data_ptr()
         if (qp | kp | vp) % 16:
