@@ -2104,76 +2104,142 @@ constexpr int kMaxSplits = 1024;
 constexpr int kAutoSplitMax = 256;
 constexpr int kAutoCausalItems = 8;
 
-// Modelled duration of a launch whose tiles' key ranges are cut into s
-// parts, in units of one key block's time on one workgroup. A work item
-// costs its key blocks plus kItemOverhead (pipeline fill and drain,
-// epilogue), an empty item (a causal part past the diagonal) almost nothing.
-// Equal items (full attention) run in ceil(items / cus) rounds; with a causal
-// mask the parts a tile sees whole do, and all items are bounded by
-// max(total / cus, longest item), which the work
-// queue, handing out the longest tiles first, comes close to. A split launch
-// adds the merge kernel: it reads every part's O and lse and writes O, at
-// kMergeBytesPerSecond, but no faster than one row's walk over its parts
-// (four part loads in flight, kMergeLatency per four), which is what bounds
-// it when the rows are few (decode shapes).
-constexpr double kItemOverhead = 1.5;
-constexpr double kEmptyItem = 0.1;
-constexpr double kMergeBytesPerSecond = 4.0e12;
-constexpr double kMergeLatency = 0.7e-6;
+// Strides of a contiguous [B, H, N, 128] tensor.
+Strides contiguous(int64_t heads, int64_t seq) { return Strides{heads * seq * HD, seq * HD, HD}; }
+
+Strides strides_of(const int64_t* s) { return Strides{s[0], s[1], s[2]}; }
+
+// Whether a buffer of nk_pad key rows n elements apart, of which the last may
+// lie past the tensor, is addressed with 32-bit byte offsets (buffer loads
+// check every offset against the real rows; the offsets of the rows past
+// them must not wrap). A ragged tail is then read in place; reading it
+// through padded copies costs a pass that reads and writes all of K and V
+// (B=8 Hq=64 Hkv=8 Nq=1 Nk=8005: 94 us of copies before a 51 us attention
+// kernel, 147 us per forward; in place 54 us).
+bool rows_in_place(int64_t n, int64_t nk_pad) {
+  const int64_t lim = kSpanLimit / (int64_t)sizeof(_Float16);
+  return n < lim && n * nk_pad < lim;
+}
+
+// Whether a launch of the automatic V^T tile runs its natural-V twin (the
+// same values bit for bit, see the table above): where every work item (a
+// tile, or a part of its key blocks) has a workgroup of its own and V is read in place, nothing then runs before the
+// attention kernel. That saves the prep launch, 3 us and V's bytes twice at
+// 4.7 TB/s, and costs the second operand read of every key block, 0.27 us a
+// block while few CUs are busy and less as they fill up (the power limit
+// sets the pace there). Fitted to both tiles over 12 to 256 tiles (V^T /
+// natural): 12 heads on one KV head, 256 keys 14.0 / 11.7 us, 512 18.5 /
+// 16.5, 1000 27.7 / 26.6, 2048 45.5 / 46.0; 16 KV heads, 3000 keys 83.3 /
+// 75.7, 4096 130.9 / 123.9; 64 heads on 8 KV heads, 1024 rows by 8192 keys
+// 242.3 / 239.5. At 256 blocks natural V was the slower one for every head
+// count (by 1.6 to 13 %), so the fit stops at kShortBlocks. Split launches:
+// 256 rows of 12 heads behind 32768 keys in 21 parts 69.0 / 66.5, behind
+// 131072 209.6 / 206.8, 512 rows of 32 heads on 8 behind 8192 in 4 parts 86.0 /
+// 81.8.
+constexpr int64_t kShortBlocks = 64;
+bool natural_is_shorter(const fa_problem* p, const KeyLayout& lay, const Strides& ks,
+                        const Strides& vs, int64_t items, int splits, int cus) {
+  const int64_t blocks = (lay.nk_pad / 128 + splits - 1) / splits;
+  if (items > cus || blocks > kShortBlocks || !rows_in_place(ks.n, lay.nk_pad) ||
+      !rows_in_place(vs.n, lay.nk_pad))
+    return false;
+  const double saved = 3.0 + (double)(p->batch * p->heads_kv * lay.nk_pad) * (2 * HD * sizeof(_Float16)) / 4.7e6;
+  return saved > 1.15 * (double)blocks * (0.27 - 0.15 * (double)items / cus);
+}
+
 // fa_merge_wide_kernel takes over from fa_merge_kernel for at most this many
 // rows with at least kMergeWideParts parts (one workgroup per row).
 constexpr int64_t kMergeWideRows = 4096;
 constexpr int kMergeWideParts = 32;
 bool merge_wide(int64_t rows, int splits) { return rows <= kMergeWideRows && splits >= kMergeWideParts; }
 
-// The model for s = 1..most parts (at most kAutoSplitMax). With a causal mask
-// it sums over a sequence's tiles, each tile for all counts at once: 15 tiles
-// and 125 counts (12 heads, 300 rows, 125 key blocks) take 5 us, where a walk
-// over the tiles for every count took 23, on every automatic launch.
+// Modelled duration of a launch whose tiles' key ranges are cut into s parts,
+// for s = 1..most (at most kAutoSplitMax), without a mask, in units of one key
+// block's time on one workgroup. A work item costs its key blocks plus
+// kItemOverhead (pipeline fill and drain, epilogue), and equal items run in
+// ceil(items / cus) rounds. A split launch
+// adds the merge kernel: it reads every part's O and lse and writes O, at
+// kMergeBytesPerSecond, but no faster than one row's walk over its parts
+// (four part loads in flight, kMergeLatency per four), which is what bounds
+// it when the rows are few.
+constexpr double kItemOverhead = 1.5;
+constexpr double kMergeBytesPerSecond = 4.0e12;
+constexpr double kMergeLatency = 0.7e-6;
 void split_costs(const fa_problem* p, const TileConfig* tile, const KeyLayout& lay, int cus, int most,
                  double (&cost)[kAutoSplitMax + 1]) {
-  const int bn = tile->keys;
-  const int64_t nbt = lay.nk_pad / bn;
-  const RowLayout rl = row_layout(p);
-  const int64_t nbh = rl.seqs, tiles_q = (rl.rows + kRows - 1) / kRows;
-  if (p->causal == FA_CAUSAL_NONE) {
-    for (int s = 1; s <= most; ++s)
-      cost[s] = ceil((double)(nbh * tiles_q) * s / cus) * ((double)((nbt + s - 1) / s) + kItemOverhead);
-  } else {
-    const int64_t off = p->causal == FA_CAUSAL_BOTTOM_RIGHT ? p->seq_k - p->seq_q : 0;
-    // Over the tiles: key blocks seen, parts seen, and parts seen by more than half.
-    int64_t sum = 0, widest = 0;
-    double seen[kAutoSplitMax + 1] = {}, half[kAutoSplitMax + 1] = {};
-    const double eps = 0.25 / (double)nbt;     // vis * s / nbt is a multiple of 1 / nbt
-    for (int64_t r = 0; r < tiles_q; ++r) {
-      // Keys [0, kend) are seen by the tile's last row (its position + 1):
-      // vis key blocks, which fill some parts and reach into one more.
-      const int64_t kend = (std::min<int64_t>((r + 1) * kRows, rl.rows) - 1) / rl.pack + 1 + off;
-      const int64_t vis = kend <= 0 ? 0 : std::min<int64_t>(nbt, (kend + bn - 1) / bn);
-      if (vis == 0) continue;
-      sum += vis;
-      widest = std::max(widest, vis);
-      const double share = (double)vis / (double)nbt;
-      for (int s = 1; s <= most; ++s) {
-        seen[s] += (double)((int)(share * s - eps) + 1);     // vis * s / nbt rounded up
-        half[s] += (double)(int)(share * s + (0.5 - eps));   // rounded, halves down
-      }
-    }
-    for (int s = 1; s <= most; ++s) {
-      const double total = (double)nbh * ((double)sum + seen[s] * kItemOverhead +
-                                          ((double)tiles_q * s - seen[s]) * kEmptyItem);
-      const double longest = (double)std::min(widest, (nbt + s - 1) / s) + (widest ? kItemOverhead : 0.0);
-      cost[s] = std::max({total / cus, longest, ceil(nbh * half[s] / cus) * (double)(nbt / s + kItemOverhead)});
-    }
-  }
+  const int64_t nbt = lay.nk_pad / tile->keys;
   const double rows = (double)(p->batch * p->heads_q) * p->seq_q;
-  for (int s = 2; s <= most; ++s) {
+  const double block_seconds = tile->keys == 128 ? 3.4e-6 : 1.8e-6;
+  for (int s = 1; s <= most; ++s) {
+    cost[s] = ceil((double)grid_size(p) * s / cus) * ((double)((nbt + s - 1) / s) + kItemOverhead);
+    if (s == 1) continue;
     const double bytes = rows * (s * (HD * 4.0 + 4.0) + HD * 2.0 + 4.0);
-    const double block_seconds = bn == 128 ? 3.4e-6 : 1.8e-6;
     // A row's walk: four part loads in flight per lane, over all its parts
     // (fa_merge_kernel) or over an eighth of them (fa_merge_wide_kernel).
     const int walk = merge_wide((int64_t)rows, s) ? (s + 7) / 8 : s;
     cost[s] += std::max(bytes / kMergeBytesPerSecond, ((walk + 3) / 4) * kMergeLatency) / block_seconds;
+  }
+}
+
+// The same with a causal mask, in us, from sums over a sequence's tiles, each
+// tile for all counts at once (15 tiles and 125 counts, of 12 heads with 300
+// rows and 125 key blocks, take 5 us; a walk over the tiles for every count
+// took 23). A key block takes 1.8 us on a CU with the others idle and 3.6 with
+// all 256 busy (the power limit): in between, by the share of the CUs that
+// the blocks keep busy while the longest item runs. The launch lasts as long
+// as its longest item, as all its blocks spread over the CUs, or as the rounds
+// of the parts that a tile sees by more than half, of which a last, partial one
+// counts 0.37 and the rest by its size. More items than CUs cost the queues'
+// reset and claims, a V^T pass its bytes (natural_is_shorter), a split the
+// merge. Fitted to 230 launches of 257 to 16000 rows per KV head with 1 to 128
+// parts each: the count it picks takes 0.4 % longer than the fastest timed
+// one there. The rounds alone, blind to the V^T pass and the busy share, were
+// 7 % behind it, and 39 % where more items than CUs bring the pass back: 3
+// causal prompts of 2329 keys, one head, 10 parts (300 items) 40.8 us, 8 (240)
+// 29.3.
+void causal_costs(const fa_problem* p, const TileConfig* tile, const KeyLayout& lay, int cus, int most,
+                  double (&cost)[kAutoSplitMax + 1]) {
+  const int bn = tile->keys;
+  const int64_t nbt = lay.nk_pad / bn;
+  const RowLayout rl = row_layout(p);
+  const int64_t nbh = rl.seqs, tiles_q = (rl.rows + kRows - 1) / kRows;
+  const int64_t off = p->causal == FA_CAUSAL_BOTTOM_RIGHT ? p->seq_k - p->seq_q : 0;
+  // Over the tiles: key blocks seen, parts seen, and parts seen by more than half.
+  int64_t sum = 0, widest = 0;
+  double seen[kAutoSplitMax + 1] = {}, half[kAutoSplitMax + 1] = {};
+  const double eps = 0.25 / (double)nbt;     // vis * s / nbt is a multiple of 1 / nbt
+  for (int64_t r = 0; r < tiles_q; ++r) {
+    // Keys [0, kend) are seen by the tile's last row (its position + 1):
+    // vis key blocks, which fill some parts and reach into one more.
+    const int64_t kend = (std::min<int64_t>((r + 1) * kRows, rl.rows) - 1) / rl.pack + 1 + off;
+    const int64_t vis = kend <= 0 ? 0 : std::min<int64_t>(nbt, (kend + bn - 1) / bn);
+    if (vis == 0) continue;
+    sum += vis;
+    widest = std::max(widest, vis);
+    const double share = (double)vis / (double)nbt;
+    for (int s = 1; s <= most; ++s) {
+      seen[s] += (double)((int)(share * s - eps) + 1);     // vis * s / nbt rounded up
+      half[s] += (double)(int)(share * s + (0.5 - eps));   // rounded, halves down
+    }
+  }
+  const double scale = bn == 128 ? 1.0 : 0.53;             // a 64-key block's time
+  auto block_us = [&](double busy) { return scale * (1.78 + 1.79 * std::min(1.0, busy / kPlanCus)); };
+  const Strides ks = contiguous(p->heads_kv, p->seq_k);
+  const double copy_us = (double)(p->batch * p->heads_kv * lay.nk_pad) * (2 * HD * sizeof(_Float16)) / 8.3e6;
+  const double rows = (double)(p->batch * p->heads_q) * p->seq_q, blocks = (double)(nbh * sum);
+  for (int s = 1; s <= most; ++s) {
+    const int64_t items = nbh * tiles_q * s;
+    const bool in_place = lay.vnat || (p->kernel == 0 && natural_is_shorter(p, lay, ks, ks, items, s, cus));
+    const double longest = (double)std::max<int64_t>(1, std::min(widest, (nbt + s - 1) / s));
+    const double block = block_us(std::min((double)cus, blocks / longest));
+    const double x = nbh * half[s] / cus, full = floor(x);
+    const double rounds = x > 0.0 && x <= 1.0 ? 1.0 : full + (x > full ? 0.37 + 0.63 * (x - full) : 0.0);
+    cost[s] = 7.2 + (in_place ? 0.0 : copy_us) + (items > cus ? 7.9 * cus / kPlanCus : 0.0) +
+              std::max({longest * block + 2.85, (blocks + 0.97 * nbh * seen[s]) / cus * block_us(cus),
+                        rounds * (std::min((double)nbt / s, longest) * block + 2.85)});
+    if (s == 1) continue;
+    const int walk = merge_wide((int64_t)rows, s) ? (s + 7) / 8 : s;
+    cost[s] += 4.5 + std::max(rows * s * (HD * 4.0 + 4.0) / 3.0e6, 0.86 * ((walk + 3) / 4));
   }
 }
 
@@ -2269,8 +2335,8 @@ SplitChoice choose_few_rows(const fa_problem* p, const KeyLayout& lay, int reque
 
 // How a split launch runs for a requested part count: 0 picks the count with
 // the shortest modelled launch (above the few-row kernel's rows, splitting
-// only when that beats one pass over the
-// keys by 10 %: tiles must leave CUs idle), n >= 1 is clamped to the tile's
+// only when that beats one pass over the keys by 10 %, without a mask: tiles
+// must leave CUs idle), n >= 1 is clamped to the tile's
 // key blocks (every part then has at least one). The resolved count requested
 // again resolves to the same choice.
 int resolve_splits(const fa_problem* p, const TileConfig* tile, const KeyLayout& lay,
@@ -2287,8 +2353,9 @@ int resolve_splits(const fa_problem* p, const TileConfig* tile, const KeyLayout&
           most, std::max<int64_t>(16, kAutoCausalItems * (int64_t)cus / (int64_t)grid_size(p)));
     most = std::min(most, nbt);
     double cost[kAutoSplitMax + 1];
-    split_costs(p, tile, lay, cus, (int)most, cost);
-    double best = 0.9 * cost[1];
+    const bool causal = p->causal != FA_CAUSAL_NONE;
+    (causal ? causal_costs : split_costs)(p, tile, lay, cus, (int)most, cost);
+    double best = (causal ? 1.0 : 0.9) * cost[1];
     for (int s = 2; s <= most; ++s)
       if (cost[s] < best) {
         best = cost[s];
@@ -2298,49 +2365,6 @@ int resolve_splits(const fa_problem* p, const TileConfig* tile, const KeyLayout&
   if ((int64_t)grid_size(p) * c.parts >= ((int64_t)1 << 30)) return FA_ERR_GEOMETRY;
   *out = c;
   return FA_OK;
-}
-
-// Strides of a contiguous [B, H, N, 128] tensor.
-Strides contiguous(int64_t heads, int64_t seq) { return Strides{heads * seq * HD, seq * HD, HD}; }
-
-Strides strides_of(const int64_t* s) { return Strides{s[0], s[1], s[2]}; }
-
-// Whether a buffer of nk_pad key rows n elements apart, of which the last may
-// lie past the tensor, is addressed with 32-bit byte offsets (buffer loads
-// check every offset against the real rows; the offsets of the rows past
-// them must not wrap). A ragged tail is then read in place; reading it
-// through padded copies costs a pass that reads and writes all of K and V
-// (B=8 Hq=64 Hkv=8 Nq=1 Nk=8005: 94 us of copies before a 51 us attention
-// kernel, 147 us per forward; in place 54 us).
-bool rows_in_place(int64_t n, int64_t nk_pad) {
-  const int64_t lim = kSpanLimit / (int64_t)sizeof(_Float16);
-  return n < lim && n * nk_pad < lim;
-}
-
-// Whether a launch of the automatic V^T tile runs its natural-V twin (the
-// same values bit for bit, see the table above): where every work item (a
-// tile, or a part of its key blocks) has a workgroup of its own and V is read in place, nothing then runs before the
-// attention kernel. That saves the prep launch, 3 us and V's bytes twice at
-// 4.7 TB/s, and costs the second operand read of every key block, 0.27 us a
-// block while few CUs are busy and less as they fill up (the power limit
-// sets the pace there). Fitted to both tiles over 12 to 256 tiles (V^T /
-// natural): 12 heads on one KV head, 256 keys 14.0 / 11.7 us, 512 18.5 /
-// 16.5, 1000 27.7 / 26.6, 2048 45.5 / 46.0; 16 KV heads, 3000 keys 83.3 /
-// 75.7, 4096 130.9 / 123.9; 64 heads on 8 KV heads, 1024 rows by 8192 keys
-// 242.3 / 239.5. At 256 blocks natural V was the slower one for every head
-// count (by 1.6 to 13 %), so the fit stops at kShortBlocks. Split launches:
-// 256 rows of 12 heads behind 32768 keys in 21 parts 69.0 / 66.5, behind
-// 131072 209.6 / 206.8, 512 rows of 32 heads on 8 behind 8192 in 4 parts 86.0 /
-// 81.8.
-constexpr int64_t kShortBlocks = 64;
-bool natural_is_shorter(const fa_problem* p, const KeyLayout& lay, const Strides& ks,
-                        const Strides& vs, int64_t items, int splits, int cus) {
-  const int64_t blocks = (lay.nk_pad / 128 + splits - 1) / splits;
-  if (items > cus || blocks > kShortBlocks || !rows_in_place(ks.n, lay.nk_pad) ||
-      !rows_in_place(vs.n, lay.nk_pad))
-    return false;
-  const double saved = 3.0 + (double)(p->batch * p->heads_kv * lay.nk_pad) * (2 * HD * sizeof(_Float16)) / 4.7e6;
-  return saved > 1.15 * (double)blocks * (0.27 - 0.15 * (double)items / cus);
 }
 
 // Caller strides must keep every 128-element row 16-byte aligned and rows

@@ -114,3 +114,15 @@ def test_operator_resolves_the_count_once(library_path):
     op(q, k, k)
     (plan,) = op.plans.values()
     assert plan.before[1] == op.split_count(q.shape, k.shape) > 1
+
+
+# (B, Hq, Hkv, Nq, Nk, mask, most parts): more items than CUs bring back the
+# pass over V and the queues; parts that many tiles cannot use only cost a merge.
+@pytest.mark.parametrize("shape,causal,most", [
+    ((3, 1, 1, 2329, 2329), "top_left", 8), ((1, 1, 1, 3589, 10404), "top_left", 17),
+    ((2, 12, 2, 576, 1104), "top_left", 1), ((3, 8, 4, 3544, 5788), "top_left", 1),
+    ((1, 64, 64, 1087, 6144), "bottom_right", 1), ((4, 2, 1, 2421, 2862), "bottom_right", 4),
+], ids=str)
+def test_causal_parts_stay_within_the_cus(library_path, shape, causal, most):
+    lib = binding.load_library(library_path)
+    assert 1 <= parts(lib, shape, causal) <= most
