@@ -870,13 +870,14 @@ __device__ __forceinline__ void fa_pp_tile(const FaArgs& args, const int tile, c
   // block past the tile's last one, an offset past any buffer's end: such a
   // load is issued like any other (which keeps the wait counts fixed) but
   // fetches nothing. (Loading the last block again in its place cost 1.5
-  // blocks of L2 traffic per tile.) The natural-V kernels that can cut tiles
-  // do load the last block again, which their loop runs faster with, most
-  // where only some waves of a group have rows: 160 rows for each of 16 KV
-  // heads behind 65536 keys in 16 parts 132.2 -> 129.0 us, 8 KV heads 76.9 ->
-  // 75.0; one-pass launches of 1000 keys lose 0.7 % by it.
+  // blocks of L2 traffic per tile.) The unpacked natural-V kernels that can cut
+  // tiles do load the last block again, which they run faster with: over 100
+  // split launches up to 8 % (64 KV heads, 358 rows behind 10600 keys, 2 parts,
+  // 177.3 -> 163.3 us; 45 of 372 rows behind 7133, 110.3 -> 101.6), where the
+  // packed ones lose as much (8 KV heads, 660 rows behind 115194 keys, 21
+  // parts, 335.7 without, 362.3 with it) and one-pass launches of 1000 keys 0.7 %.
   const int last = nblk - 1;
-  constexpr bool CLAMP = VNAT && can_cut(MODE);
+  constexpr bool CLAMP = VNAT && !PACKED && can_cut(MODE);
   constexpr uint32_t NOWHERE = (uint32_t)kSpanLimit;
   auto offset = [&](int b, int bytes) {
     return CLAMP ? (uint32_t)(min(b, last) * bytes) : b <= last ? (uint32_t)(b * bytes) : NOWHERE;
