@@ -354,7 +354,8 @@ int fa_fwd_split(const fa_problem* p, int32_t splits, const fa_strides* strides,
  * to 256 (work items per CU, per-item overhead, the merge's HBM traffic or,
  * with few rows, its walk over the parts; for at most 4096 rows and 32 parts
  * or more the merge gives each row a workgroup) and splits only when that
- * beats one pass over the keys by 10 %; for at most 256 rows per KV head it
+ * beats one pass over the keys by 10 % (with a causal mask, where the model
+ * is a finer one, by any margin); for at most 256 rows per KV head it
  * compares the counts of both kernels (see above) with one pass. The count
  * returned, requested again, runs the same launch without the search. */
 
